@@ -60,6 +60,9 @@ constexpr uint32_t Kind_error = 5;
 
 constexpr float Flt_max = 3.40282347e+38f;
 
+// bit of the error word that is no error: a vertex is not finite
+constexpr uint32_t Not_finite = 16;
+
 // scene::bvh::Reference: {min.xyz, primitive}{max.xyz, pad}
 struct Ref {
     float    lo[3];
@@ -231,13 +234,18 @@ __global__ void make_refs(float const* __restrict__ positions, uint32_t stride,
         float const* pb = positions + size_t(ib) * stride;
         float const* pc = positions + size_t(ic) * stride;
 
-        Ref r;
+        Ref  r;
+        bool finite = true;
         for (int i = 0; i < 3; ++i) {
             // triangle_bvh_helper.cpp:15-21: min(a, min(b, c))
             r.lo[i] = smin(pa[i], smin(pb[i], pc[i]));
             r.hi[i] = smax(pa[i], smax(pb[i], pc[i]));
             lo[i]   = r.lo[i];
             hi[i]   = r.hi[i];
+            finite  = finite && isfinite(pa[i]) && isfinite(pb[i]) && isfinite(pc[i]);
+        }
+        if (!finite) {
+            atomicOr(error, Not_finite);
         }
         r.prim  = t;
         r.pad   = 0;
@@ -1356,7 +1364,7 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
         if (err & 4u) {
             return fail(MI_ERR_HIP, "mi_bvh_build: internal error (side counts)");
         }
-        if (err) {
+        if (err & ~Not_finite) {
             return fail(MI_ERR_UNSPLITTABLE,
                         "mi_bvh_build: a node of more than 255 references cannot be split "
                         "(level %zu)",
@@ -1473,10 +1481,11 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
         bvh.release();
         return fail(MI_ERR_HIP, "bvh build: %s", hipGetErrorString(e));
     }
-    if (err) {
+    if (err & ~Not_finite) {
         bvh.release();
-        return fail(MI_ERR_HIP, "mi_bvh_build: internal error (layout %u)", err);
+        return fail(MI_ERR_HIP, "mi_bvh_build: internal error (layout %u)", err & ~Not_finite);
     }
+    bvh.nan_bounds = 0 != (err & Not_finite);
     for (int a = 0; a < 3; ++a) {
         bvh.aabb_min[a] = root[a];
         bvh.aabb_max[a] = root[4 + a];

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -114,8 +115,12 @@ int32_t upload_bvh(void const* nodes, uint32_t num_nodes, uint32_t const* slots,
     // bounds the stack a traversal needs even for a shared child.
     std::vector<uint32_t> depth(num_nodes, 0);
     uint32_t              max_depth = 0;
+    bool                  finite    = true;
     for (uint32_t i = 0; i < num_nodes; ++i) {
         HostNode const& n = hn[i];
+        for (int k = 0; k < 3; ++k) {
+            finite = finite && std::isfinite(n.lo[k]) && std::isfinite(n.hi[k]);
+        }
         if (0 == n.num) {
             if (n.axis > 2 || n.data <= i || uint64_t(n.data) + 1 >= num_nodes) {
                 return fail(MI_ERR_ARGS, "node %u: bad children %u (axis %u)", i, n.data, n.axis);
@@ -145,6 +150,7 @@ int32_t upload_bvh(void const* nodes, uint32_t num_nodes, uint32_t const* slots,
     bvh.num_slots     = num_slots;
     bvh.num_triangles = num_triangles;
     bvh.max_depth     = max_depth;
+    bvh.nan_bounds    = !finite;
     for (int k = 0; k < 3; ++k) {
         bvh.aabb_min[k] = hn[0].lo[k];
         bvh.aabb_max[k] = hn[0].hi[k];

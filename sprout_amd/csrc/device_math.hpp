@@ -109,6 +109,29 @@ __device__ __forceinline__ bool slab_entry(float4 lo, float4 hi, F3 o, F3 inv, f
     return (tmax >= min_t) & (max_t >= tmin) & (tmax >= tmin);
 }
 
+// slab_entry without the per-coordinate NaN filters, for boxes without NaN
+// coordinates.  A coordinate product is NaN then only where the ray's
+// inverse direction or origin is (both ends of the axis alike, dropped by
+// min / max as the filter drops them; with all three axes gone the negated
+// comparisons below admit the box as the filtered infinities do), or
+// where an infinite origin meets an infinite bound, a ray no triangle
+// accepts.  24 operations a box instead of 36; tmin may be NaN (all axes
+// gone) and compares as -infinity through !(max_t < tmin).
+__device__ __forceinline__ bool slab_lean(float4 lo, float4 hi, F3 o, F3 inv, float min_t,
+                                          float max_t, float& tmin_out) {
+    float const l1x = (lo.x - o.x) * inv.x;
+    float const l1y = (lo.y - o.y) * inv.y;
+    float const l1z = (lo.z - o.z) * inv.z;
+    float const l2x = (hi.x - o.x) * inv.x;
+    float const l2y = (hi.y - o.y) * inv.y;
+    float const l2z = (hi.z - o.z) * inv.z;
+
+    float const tmax = fminf(fminf(fmaxf(l1x, l2x), fmaxf(l1y, l2y)), fmaxf(l1z, l2z));
+    float const tmin = fmaxf(fmaxf(fminf(l1x, l2x), fminf(l1y, l2y)), fminf(l1z, l2z));
+    tmin_out         = tmin;
+    return !(tmax < min_t) & !(max_t < tmin) & !(tmax < tmin);
+}
+
 // triangle::intersect (core/scene/shape/triangle/triangle_primitive_mt.inl:61-93)
 // with e1 = b - a and e2 = c - a precomputed (the same rounded subtraction).
 // On a hit returns true and sets t, u, v.

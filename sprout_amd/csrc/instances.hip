@@ -267,165 +267,113 @@ __device__ __forceinline__ void unpack_node(uint32_t e, uint32_t& data, uint32_t
     meta = ((e >> Data_bits) & 3u) | ((e >> 24) << 8);
 }
 
+// Entries {node word, entry distance} of eight bytes.
 struct Pair_stack {
-    uint32_t* lds;    // 2 * Lds_entries * Block2 words, entry-major
-    uint32_t* spill;  // 2 * spill entries * total words, entry-major
+    uint2*    lds;    // Lds_entries * Block2 entries, entry-major
+    uint64_t* spill;  // spill entries * total entries, entry-major
     uint32_t  gid;
     uint32_t  total;
     uint32_t  sp;
 
-    __device__ void push(uint32_t node, float tmin) {
+    __device__ __forceinline__ void push(uint32_t node, float tmin) {
         if (sp < Lds_entries) {
-            lds[(2 * sp) * Block2 + threadIdx.x]     = node;
-            lds[(2 * sp + 1) * Block2 + threadIdx.x] = __float_as_uint(tmin);
+            lds[sp * Block2 + threadIdx.x] = make_uint2(node, __float_as_uint(tmin));
         } else {
-            size_t const k                  = 2 * size_t(sp - Lds_entries);
-            spill[k * total + gid]       = node;
-            spill[(k + 1) * total + gid] = __float_as_uint(tmin);
+            spill[size_t(sp - Lds_entries) * total + gid] =
+                uint64_t(node) | (uint64_t(__float_as_uint(tmin)) << 32);
         }
         ++sp;
     }
 
-    __device__ void pop(uint32_t& node, float& tmin) {
+    __device__ __forceinline__ void pop(uint32_t& node, float& tmin) {
         --sp;
         if (sp < Lds_entries) {
-            node = lds[(2 * sp) * Block2 + threadIdx.x];
-            tmin = __uint_as_float(lds[(2 * sp + 1) * Block2 + threadIdx.x]);
+            uint2 const e = lds[sp * Block2 + threadIdx.x];
+            node          = e.x;
+            tmin          = __uint_as_float(e.y);
         } else {
-            size_t const k = 2 * size_t(sp - Lds_entries);
-            node           = spill[k * total + gid];
-            tmin           = __uint_as_float(spill[(k + 1) * total + gid]);
+            // atomic, so that the branches' loads are not merged into a flat one
+            uint64_t const e = __hip_atomic_load(&spill[size_t(sp - Lds_entries) * total + gid],
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SINGLETHREAD);
+            node             = uint32_t(e);
+            tmin             = __uint_as_float(uint32_t(e >> 32));
         }
     }
 };
 
-// Pops until a pending child passes its box test; false at a sentinel (which
-// is consumed) or an empty stack.
-__device__ __forceinline__ bool pop_pending(Pair_stack& stack, Iray const& r, uint32_t& data,
-                                            uint32_t& meta) {
+enum Popped { Pop_done = 0, Pop_node = 1, Pop_sentinel = 2 };
+
+// Pops until a pending child passes its box test, a sentinel (which is
+// consumed) comes up, or the stack is empty.
+__device__ __forceinline__ Popped pop_pending(Pair_stack& stack, float max_t, uint32_t& data,
+                                              uint32_t& meta) {
     while (stack.sp > 0) {
         uint32_t e;
         float    tmin;
         stack.pop(e, tmin);
         if (Sentinel_word == e) {
-            return false;
+            return Pop_sentinel;
         }
-        if (r.max_t >= tmin) {
+        if (!(max_t < tmin)) {
             unpack_node(e, data, meta);
-            return true;
+            return Pop_node;
         }
+    }
+    return Pop_done;
+}
+
+// One inner node of either level (node data = first of the sibling pair);
+// false when neither child is hit.
+__device__ __forceinline__ bool pair_step(float4 const* __restrict__ nodes, Pair_stack& stack,
+                                          Iray const& r, uint32_t& data, uint32_t& meta) {
+    float4 const* const pair = nodes + 2 * size_t(data);
+    float4 const        alo = pair[0];
+    float4 const        ahi = pair[1];
+    float4 const        blo = pair[2];
+    float4 const        bhi = pair[3];
+    float               ta, tb;
+    bool const          ha   = dev::slab_lean(alo, ahi, r.o, r.inv, r.min_t, r.max_t, ta);
+    bool const          hb   = dev::slab_lean(blo, bhi, r.o, r.inv, r.min_t, r.max_t, tb);
+    bool const          flip = 0 != ((r.sign_bits >> node_axis(meta)) & 1u);
+    bool const          both = ha & hb;
+    bool const          take_b = (both & flip) | (hb & !ha);
+    if (both) {
+        stack.push(pack_node(__float_as_uint(take_b ? alo.w : blo.w),
+                             __float_as_uint(take_b ? ahi.w : bhi.w)),
+                   take_b ? ta : tb);
+    }
+    if (ha | hb) {
+        data = __float_as_uint(take_b ? blo.w : alo.w);
+        meta = __float_as_uint(take_b ? bhi.w : ahi.w);
+        return true;
     }
     return false;
 }
 
-// One inner node of either level (node data = first of the sibling pair).
-__device__ __forceinline__ bool pair_step(float4 const* __restrict__ nodes, Pair_stack& stack,
-                                          Iray const& r, uint32_t& data, uint32_t& meta) {
-    uint32_t const a   = data;
-    float4 const   alo = nodes[2 * size_t(a) + 0];
-    float4 const   ahi = nodes[2 * size_t(a) + 1];
-    float4 const   blo = nodes[2 * size_t(a) + 2];
-    float4 const   bhi = nodes[2 * size_t(a) + 3];
-    float          ta, tb;
-    bool const     ha   = dev::slab_entry(alo, ahi, r.o, r.inv, r.min_t, r.max_t, ta);
-    bool const     hb   = dev::slab_entry(blo, bhi, r.o, r.inv, r.min_t, r.max_t, tb);
-    bool const     flip = (r.sign_bits >> node_axis(meta)) & 1u;
-    bool const     hn   = flip ? hb : ha;
-    bool const     hf   = flip ? ha : hb;
-    if (hn | hf) {
-        if (hn & hf) {
-            stack.push(pack_node(__float_as_uint(flip ? alo.w : blo.w),
-                                 __float_as_uint(flip ? ahi.w : bhi.w)),
-                       flip ? ta : tb);
-        }
-        bool const take_b = hn ? flip : !flip;
-        data              = __float_as_uint(take_b ? blo.w : alo.w);
-        meta              = __float_as_uint(take_b ? bhi.w : ahi.w);
-        return true;
-    }
-    return pop_pending(stack, r, data, meta);
-}
-
-// Tree::intersect / intersect_p of one mesh above a sentinel; returns with
-// the sentinel popped.  Closest: shrinks r.max_t on every hit.
-template <bool Any>
-__device__ bool mesh_pairs(float4 const* __restrict__ nodes, float4 const* __restrict__ tris,
-                           Iray& r, Pair_stack& stack, uint32_t& index, uint32_t& slot, float& u,
-                           float& v) {
-    stack.push(Sentinel_word, 0.f);
-    bool         hit  = false;
-    float4 const rlo  = nodes[0];
-    float4 const rhi  = nodes[1];
-    uint32_t     data = __float_as_uint(rlo.w);
-    uint32_t     meta = __float_as_uint(rhi.w);
-    bool         live = dev::slab(rlo, rhi, r.o, r.inv, r.min_t, r.max_t);
-    if (!live) {
-        uint32_t e;
-        float    t;
-        stack.pop(e, t);  // the sentinel
-        return false;
-    }
-    while (live) {
-        uint32_t const num = node_num(meta);
-        if (0 == num) {
-            live = pair_step(nodes, stack, r, data, meta);
-            continue;
-        }
-        for (uint32_t i = data, end = data + num; i < end; ++i) {
-            float4 const ta = tris[3 * size_t(i) + 0];
-            float4 const t1 = tris[3 * size_t(i) + 1];
-            float4 const t2 = tris[3 * size_t(i) + 2];
-            float        t, tu, tv;
-            if (dev::triangle({ta.x, ta.y, ta.z}, {t1.x, t1.y, t1.z}, {t2.x, t2.y, t2.z}, r.o, r.d,
-                              r.min_t, r.max_t, t, tu, tv)) {
-                hit = true;
-                if (Any) {
-                    // unwind to the sentinel
-                    uint32_t e;
-                    float    tm;
-                    do {
-                        stack.pop(e, tm);
-                    } while (Sentinel_word != e);
-                    return true;
-                }
-                r.max_t = t;
-                u       = tu;
-                v       = tv;
-                index   = __float_as_uint(ta.w);
-                slot    = i;
-            }
-        }
-        live = pop_pending(stack, r, data, meta);
-    }
-    return hit;
-}
-
 // The two-level traversal with the two-word stack as a persistent kernel
-// with per-lane ray refill: each lane walks its ray as a small state machine
-// (a top-level node, the instances of a top-level leaf in slot order, or a
-// node of an instance's mesh above a sentinel), one step per loop turn, and
-// takes a new ray when its ray is done, so a wave's lanes stay busy while
-// rays of very different lengths finish (one ray per lane for the whole walk
-// ran 0.54 Grays/s on 64 instances; this runs 1.49).  Each ray visits nodes,
-// instances and triangles in the reference's order; waves claim rays from
-// spread counters (Claims).
+// with per-lane ray refill.  A lane is at an inner node of either level, at a
+// triangle of a mesh leaf, or at an instance of a top-level leaf, and one turn
+// of the loop is one step of the kind that most of the wave's lanes wait for
+// (as trace_refill_packed; one step of every lane's own kind per turn, with
+// the two levels' inner nodes apart, ran 1.0 M rays into 64 instances in 850
+// us).  The levels share one ray in registers: an instance step reads the
+// world ray again and leaves it, or the object ray of the instance entered, as
+// the lane's ray; max_t is the same along both.  Each ray visits nodes,
+// instances and triangles in the reference's order; waves take rays as Claims
+// hands them out.
 constexpr uint32_t Refill_lanes = 8;   // refill once this many lanes of a wave are idle
 constexpr uint32_t Claim_batch  = 64;  // rays a wave claims per atomic
-
-constexpr uint32_t Phase_top  = 0;  // at a node of the top-level tree
-constexpr uint32_t Phase_leaf = 1;  // box-testing the instances of a top-level leaf
-constexpr uint32_t Phase_mesh = 2;  // at a node of an instance's mesh tree
 
 template <bool Any>
 __global__ void __launch_bounds__(Block2) trace_instances_refill(Tlas_view t, uint32_t* spill,
                                                                  uint32_t total, uint32_t* counters,
                                                                  mi_ray const* rays, uint32_t num_rays,
                                                                  uint32_t const* num_rays_dev,
-                                                                 void* out) {
-    __shared__ uint32_t lds[2 * Lds_entries * Block2];
-    Pair_stack          stack;
+                                                                 uint32_t spread, void* out) {
+    __shared__ uint2 lds[Lds_entries * Block2];
+    Pair_stack       stack;
     stack.lds   = lds;
-    stack.spill = spill;
+    stack.spill = reinterpret_cast<uint64_t*>(spill);
     stack.gid   = blockIdx.x * blockDim.x + threadIdx.x;
     stack.total = total;
     stack.sp    = 0;
@@ -433,33 +381,44 @@ __global__ void __launch_bounds__(Block2) trace_instances_refill(Tlas_view t, ui
     if (num_rays_dev) {
         num_rays = min(num_rays, *num_rays_dev);
     }
-    uint32_t const lane    = threadIdx.x & 63;
-    uint64_t const lt_mask = (uint64_t(1) << lane) - 1;
+    uint32_t const lane = threadIdx.x & 63;
 
-    Claims claims;
-    claims.init();
+    Claims   claims;
     bool     active    = false;
     bool     exhausted = false;
-    uint32_t pool_next = 0;
-    uint32_t pool_end  = 0;
+    uint32_t pool_next;
+    uint32_t pool_end;
+    claims.init(__builtin_amdgcn_readfirstlane(stack.gid >> 6), (gridDim.x * blockDim.x) >> 6, spread,
+                num_rays, pool_next, pool_end);
 
-    uint32_t      r     = 0;
-    uint32_t      phase = Phase_top;
-    Iray          w, o;
+    uint32_t      r       = 0;
+    bool          in_mesh = false;  // below a sentinel
+    bool          at_inst = false;  // at an instance of a top-level leaf
+    Iray          c;                // the ray of the lane's level
     uint32_t      data = 0, meta = 0;
-    uint32_t      leaf_i = 0, leaf_end = 0;
+    uint32_t      leaf_data = 0, leaf_meta = 0;  // the top-level leaf's instances left
     uint32_t      inst   = Null;
-    float4 const* mnodes = nullptr;
+    float4 const* nodes  = t.nodes;
     float4 const* mtris  = nullptr;
     uint32_t      instance = Null, index = Null, slot = Null;
     float         u = 0.f, v = 0.f;
 
+    auto world_ray = [&](uint32_t k) {
+        float4 const* rp = reinterpret_cast<float4 const*>(rays) + 2 * size_t(k);
+        float4 const  ro = rp[0];
+        float4 const  rd = rp[1];
+        c.o              = {ro.x, ro.y, ro.z};
+        c.min_t          = ro.w;
+        c.d              = {rd.x, rd.y, rd.z};
+        set_inverse(c);
+        return rd.w;
+    };
     auto finish = [&](bool any) {
         if (Any) {
             static_cast<uint32_t*>(out)[r] = any ? 1u : 0u;
         } else {
             mi_instance_hit h;
-            h.t        = w.max_t;
+            h.t        = c.max_t;
             h.u        = Null != index ? u : 0.f;
             h.v        = Null != index ? v : 0.f;
             h.triangle = index;
@@ -470,18 +429,35 @@ __global__ void __launch_bounds__(Block2) trace_instances_refill(Tlas_view t, ui
         }
         active = false;
     };
+    // the next pending node, the instances left of the top-level leaf whose
+    // mesh is done, or the end of the ray
+    auto next = [&]() {
+        Popped const p = pop_pending(stack, c.max_t, data, meta);
+        if (Pop_done == p) {
+            finish(false);
+        } else if (Pop_sentinel == p) {
+            in_mesh = false;
+            at_inst = true;
+        } else {
+            at_inst = !in_mesh & (0 != node_num(meta));
+            if (at_inst) {
+                leaf_data = data;
+                leaf_meta = meta;
+            }
+        }
+    };
 
     for (;;) {
-        uint64_t       idle   = __ballot(!active);
-        uint32_t const n_idle = uint32_t(__popcll(idle));
-        if ((n_idle >= Refill_lanes || 64 == n_idle) && !(exhausted && pool_next >= pool_end)) {
+        uint64_t live   = __ballot(active);
+        uint32_t n_live = uint32_t(__popcll(live));
+        if ((64 - n_live >= Refill_lanes || 0 == n_live) && !(exhausted && pool_next >= pool_end)) {
+            uint64_t idle = ~live;
             while (idle) {
                 if (pool_next >= pool_end) {
                     if (exhausted) {
                         break;
                     }
-                    uint32_t const leader = uint32_t(__ffsll(static_cast<unsigned long long>(idle))) - 1;
-                    if (!claims.next(counters, num_rays, Claim_batch, lane, leader, pool_next, pool_end)) {
+                    if (!claims.next(counters, num_rays, Claim_batch, lane, pool_next, pool_end)) {
                         exhausted = true;
                         break;
                     }
@@ -490,28 +466,26 @@ __global__ void __launch_bounds__(Block2) trace_instances_refill(Tlas_view t, ui
                 uint32_t const want  = uint32_t(__popcll(idle));
                 uint32_t const take  = avail < want ? avail : want;
                 bool const     mine  = (idle >> lane) & 1u;
-                uint32_t const rank  = uint32_t(__popcll(idle & lt_mask));
+                uint32_t const rank  = __builtin_amdgcn_mbcnt_hi(
+                    uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
                 if (mine && rank < take) {
-                    r                = pool_next + rank;
-                    float4 const* rp = reinterpret_cast<float4 const*>(rays) + 2 * size_t(r);
-                    float4 const  ro = rp[0];
-                    float4 const  rd = rp[1];
-                    w.o              = {ro.x, ro.y, ro.z};
-                    w.min_t          = ro.w;
-                    w.d              = {rd.x, rd.y, rd.z};
-                    w.max_t          = rd.w;
-                    set_inverse(w);
+                    r       = pool_next + rank;
+                    c.max_t = world_ray(r);
                     instance = index = slot = Null;
                     u = v    = 0.f;
                     stack.sp = 0;
-                    phase    = Phase_top;
-                    active   = false;
+                    in_mesh  = false;
+                    at_inst  = false;
+                    nodes    = t.nodes;
                     if (t.num_nodes) {
                         float4 const rlo = t.nodes[0];
                         float4 const rhi = t.nodes[1];
                         data             = __float_as_uint(rlo.w);
                         meta             = __float_as_uint(rhi.w);
-                        active           = dev::slab(rlo, rhi, w.o, w.inv, w.min_t, w.max_t);
+                        active           = dev::slab(rlo, rhi, c.o, c.inv, c.min_t, c.max_t);
+                        at_inst          = 0 != node_num(meta);
+                        leaf_data        = data;
+                        leaf_meta        = meta;
                     }
                     if (!active) {
                         finish(false);
@@ -520,96 +494,93 @@ __global__ void __launch_bounds__(Block2) trace_instances_refill(Tlas_view t, ui
                 pool_next += take;
                 idle = __ballot(mine && rank >= take);
             }
+            n_live = uint32_t(__popcll(__ballot(active)));
         }
 
-        if (0 == __ballot(active)) {
+        if (0 == n_live) {
             if (exhausted && pool_next >= pool_end) {
                 break;
             }
             continue;
         }
-        if (!active) {
-            continue;
-        }
 
-        if (Phase_top == phase) {
-            if (0 == node_num(meta)) {
-                if (!pair_step(t.nodes, stack, w, data, meta)) {
-                    finish(false);
+        bool const     inst_lane = active & at_inst;
+        bool const     leaf_lane = active & !at_inst & (0 != node_num(meta));
+        uint32_t const n_inst    = uint32_t(__popcll(__ballot(inst_lane)));
+        uint32_t const n_leaf    = uint32_t(__popcll(__ballot(leaf_lane)));
+        uint32_t const n_inner   = n_live - n_inst - n_leaf;
+
+        if (n_inner >= n_inst && n_inner >= n_leaf) {
+            if (active & !inst_lane & !leaf_lane) {
+                if (!pair_step(nodes, stack, c, data, meta)) {
+                    next();
+                } else if (!in_mesh & (0 != node_num(meta))) {
+                    at_inst   = true;
+                    leaf_data = data;
+                    leaf_meta = meta;
                 }
-            } else {
-                leaf_i   = data;
-                leaf_end = data + node_num(meta);
-                phase    = Phase_leaf;
             }
-        } else if (Phase_leaf == phase) {
-            if (leaf_i < leaf_end) {
-                uint32_t const         p  = __float_as_uint(t.slots[3 * size_t(leaf_i)].w);
-                Instance_record const& ir = t.instances[p];
-                ++leaf_i;
-                float4 const blo = make_float4(ir.lo[0], ir.lo[1], ir.lo[2], 0.f);
-                float4 const bhi = make_float4(ir.hi[0], ir.hi[1], ir.hi[2], 0.f);
-                // Prop::intersect: the prop's world box first
-                if (dev::slab(blo, bhi, w.o, w.inv, w.min_t, w.max_t)) {
-                    o.o     = xform_point(ir.world_to_object, w.o);
-                    o.d     = xform_vector(ir.world_to_object, w.d);
-                    o.min_t = w.min_t;
-                    o.max_t = w.max_t;
-                    set_inverse(o);
-                    Mesh_view const mv  = t.meshes[ir.mesh];
-                    float4 const    rlo = mv.nodes[0];
-                    float4 const    rhi = mv.nodes[1];
-                    if (dev::slab(rlo, rhi, o.o, o.inv, o.min_t, o.max_t)) {
-                        stack.push(Sentinel_word, 0.f);
-                        mnodes = mv.nodes;
-                        mtris  = mv.tris;
-                        inst   = p;
-                        data   = __float_as_uint(rlo.w);
-                        meta   = __float_as_uint(rhi.w);
-                        phase  = Phase_mesh;
-                    }
-                }
-            } else if (pop_pending(stack, w, data, meta)) {
-                phase = Phase_top;
-            } else {
-                finish(false);
-            }
-        } else {
-            uint32_t const num  = node_num(meta);
-            bool           live = true;
-            if (0 == num) {
-                live = pair_step(mnodes, stack, o, data, meta);
-            } else {
-                bool occluded = false;
-                for (uint32_t i = data, end = data + num; i < end; ++i) {
-                    float4 const ta = mtris[3 * size_t(i) + 0];
-                    float4 const t1 = mtris[3 * size_t(i) + 1];
-                    float4 const t2 = mtris[3 * size_t(i) + 2];
-                    float        th, tu, tv;
-                    if (dev::triangle({ta.x, ta.y, ta.z}, {t1.x, t1.y, t1.z}, {t2.x, t2.y, t2.z}, o.o,
-                                      o.d, o.min_t, o.max_t, th, tu, tv)) {
-                        if (Any) {
-                            occluded = true;
-                            break;
-                        }
-                        o.max_t  = th;
+        } else if (n_leaf >= n_inst) {
+            if (leaf_lane) {
+                float4 const ta = mtris[3 * size_t(data) + 0];
+                float4 const t1 = mtris[3 * size_t(data) + 1];
+                float4 const t2 = mtris[3 * size_t(data) + 2];
+                float        th, tu, tv;
+                bool         occluded = false;
+                if (dev::triangle({ta.x, ta.y, ta.z}, {t1.x, t1.y, t1.z}, {t2.x, t2.y, t2.z}, c.o, c.d,
+                                  c.min_t, c.max_t, th, tu, tv)) {
+                    if (Any) {
+                        occluded = true;
+                    } else {
+                        c.max_t  = th;
                         u        = tu;
                         v        = tv;
                         index    = __float_as_uint(ta.w);
-                        slot     = i;
+                        slot     = data;
                         instance = inst;
                     }
                 }
+                ++data;
+                meta -= 0x100u;
                 if (Any && occluded) {
                     finish(true);
-                    continue;
+                } else if (0 == node_num(meta)) {
+                    next();
                 }
-                live = pop_pending(stack, o, data, meta);
             }
-            if (!live) {
-                // the mesh's sentinel is popped: back to the leaf's next instance
-                w.max_t = o.max_t;
-                phase   = Phase_leaf;
+        } else if (inst_lane) {
+            // back at the top level, or already there: the world ray
+            world_ray(r);
+            nodes = t.nodes;
+            if (0 == node_num(leaf_meta)) {
+                at_inst = false;
+                next();
+            } else {
+                uint32_t const         p  = __float_as_uint(t.slots[3 * size_t(leaf_data)].w);
+                Instance_record const& ir = t.instances[p];
+                ++leaf_data;
+                leaf_meta -= 0x100u;
+                float4 const blo = make_float4(ir.lo[0], ir.lo[1], ir.lo[2], 0.f);
+                float4 const bhi = make_float4(ir.hi[0], ir.hi[1], ir.hi[2], 0.f);
+                // Prop::intersect: the prop's world box first
+                if (dev::slab(blo, bhi, c.o, c.inv, c.min_t, c.max_t)) {
+                    c.o = xform_point(ir.world_to_object, c.o);
+                    c.d = xform_vector(ir.world_to_object, c.d);
+                    set_inverse(c);
+                    Mesh_view const mv  = t.meshes[ir.mesh];
+                    float4 const    rlo = mv.nodes[0];
+                    float4 const    rhi = mv.nodes[1];
+                    if (dev::slab(rlo, rhi, c.o, c.inv, c.min_t, c.max_t)) {
+                        stack.push(Sentinel_word, 0.f);
+                        nodes   = mv.nodes;
+                        mtris   = mv.tris;
+                        inst    = p;
+                        data    = __float_as_uint(rlo.w);
+                        meta    = __float_as_uint(rhi.w);
+                        in_mesh = true;
+                        at_inst = false;
+                    }
+                }
             }
         }
     }
@@ -737,9 +708,9 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
 
     // the two-word stack traversal: every tree's node words must pack, and
     // the deepest stack beyond its LDS part spills to a per-thread area
-    bool packs = out.tree.num_nodes < (1u << Data_bits) && out.tree.num_slots < (1u << Data_bits);
+    bool packs = !out.tree.nan_bounds && out.tree.num_nodes < (1u << Data_bits) && out.tree.num_slots < (1u << Data_bits);
     for (uint32_t k = 0; k < num_meshes; ++k) {
-        packs = packs && meshes[k]->num_nodes < (1u << Data_bits) &&
+        packs = packs && !meshes[k]->nan_bounds && meshes[k]->num_nodes < (1u << Data_bits) &&
                 meshes[k]->num_slots < (1u << Data_bits);
     }
     if (packs) {
@@ -766,15 +737,19 @@ int32_t trace_instances_launch(Tlas const& t, uint32_t num_cus, mi_ray const* ra
     }
     Tlas_view const v = tlas_view(t);
     if (t.spill) {
-        uint64_t const wanted = (uint64_t(n) + Block2 - 1) / Block2;
+        // a small launch fills four waves per SIMD first (TraceResources::spread_waves)
+        uint32_t const spread = num_cus * 16;
+        uint64_t const want   = (uint64_t(n) + spread - 1) / spread;
+        uint64_t const chunk  = std::min<uint64_t>(want, 64);
+        uint64_t const wanted = (uint64_t(n) + chunk - 1) / chunk;
         uint32_t const blocks = uint32_t(std::min<uint64_t>(wanted, t.spill_total / Block2));
         hipLaunchKernelGGL(reset_claims, dim3(1), dim3(64), 0, stream, t.claims);
         if (any_hit) {
             hipLaunchKernelGGL(trace_instances_refill<true>, dim3(blocks), dim3(Block2), 0, stream, v,
-                               t.spill, t.spill_total, t.claims, rays, n, n_dev, out);
+                               t.spill, t.spill_total, t.claims, rays, n, n_dev, spread, out);
         } else {
             hipLaunchKernelGGL(trace_instances_refill<false>, dim3(blocks), dim3(Block2), 0, stream, v,
-                               t.spill, t.spill_total, t.claims, rays, n, n_dev, out);
+                               t.spill, t.spill_total, t.claims, rays, n, n_dev, spread, out);
         }
         if (hipError_t const e = hipGetLastError(); e) {
             return fail(MI_ERR_HIP, "instance trace: %s", hipGetErrorString(e));

@@ -106,6 +106,7 @@ struct Launch {
     uint32_t*     counter;     // claim counters of trace_refill: Claim_parts words, Claim_stride apart
     uint32_t      refill_lanes;
     uint32_t      claim_batch;
+    uint32_t      spread_waves;
     uint32_t const* order;    // kernels 3 and 4: the k-th claimed ray is order[k] (or k)
 };
 
@@ -430,11 +431,12 @@ __global__ void trace_refill(Launch p) {
     uint32_t const num_rays = p.num_rays_dev ? *p.num_rays_dev : p.num_rays;
 
     Claims   claims;
-    claims.init();
     bool     active    = false;
-    bool     exhausted = false;  // the global counter is past the last ray (wave-uniform)
-    uint32_t pool_next = 0;      // wave-uniform pool of claimed rays [pool_next, pool_end)
-    uint32_t pool_end  = 0;
+    bool     exhausted = false;  // every part is used up (wave-uniform)
+    uint32_t pool_next;          // wave-uniform pool of claimed rays [pool_next, pool_end)
+    uint32_t pool_end;
+    claims.init(__builtin_amdgcn_readfirstlane(stack.gid >> 6), p.total_threads >> 6, p.spread_waves,
+                num_rays, pool_next, pool_end);
     uint32_t r         = 0;
     Ray      ray;
     uint32_t data  = 0;
@@ -453,10 +455,7 @@ __global__ void trace_refill(Launch p) {
                     if (exhausted) {
                         break;
                     }
-                    uint32_t const leader =
-                        uint32_t(__ffsll(static_cast<unsigned long long>(idle))) - 1;
-                    if (!claims.next(p.counter, num_rays, p.claim_batch, lane, leader, pool_next,
-                                     pool_end)) {
+                    if (!claims.next(p.counter, num_rays, p.claim_batch, lane, pool_next, pool_end)) {
                         exhausted = true;
                         break;
                     }
@@ -544,9 +543,11 @@ __device__ __forceinline__ void unpack_node(uint32_t e, uint32_t& data, uint32_t
     meta = ((e >> Packed_data_bits) & 3u) | ((e >> 24) << 8);
 }
 
+// Entries {node word, entry distance} of eight bytes, entry-major: the first
+// lds_entries of a lane in LDS, deeper ones in the per-thread global area.
 struct Stack2 {
-    uint32_t* lds;          // 2 * lds_entries * block_size words, entry-major
-    uint32_t* spill;        // 2 * spill entries * total_threads words, entry-major
+    uint2*    lds;
+    uint64_t* spill;
     uint32_t  lds_entries;
     uint32_t  lane;
     uint32_t  block_size;
@@ -556,8 +557,8 @@ struct Stack2 {
 
     __device__ void init(uint32_t* lds_base, uint32_t* spill_base, uint32_t entries,
                          uint32_t threads) {
-        lds           = lds_base;
-        spill         = spill_base;
+        lds           = reinterpret_cast<uint2*>(lds_base);
+        spill         = reinterpret_cast<uint64_t*>(spill_base);
         lds_entries   = entries;
         lane          = threadIdx.x;
         block_size    = blockDim.x;
@@ -566,27 +567,30 @@ struct Stack2 {
         sp            = 0;
     }
 
-    __device__ void push(uint32_t node, float tmin) {
+    __device__ __forceinline__ void push(uint32_t node, float tmin) {
         if (sp < lds_entries) {
-            lds[(2 * sp) * block_size + lane]     = node;
-            lds[(2 * sp + 1) * block_size + lane] = __float_as_uint(tmin);
+            lds[__umul24(sp, block_size) + lane] = make_uint2(node, __float_as_uint(tmin));
         } else {
-            size_t const k                                 = 2 * size_t(sp - lds_entries);
-            spill[k * total_threads + gid]       = node;
-            spill[(k + 1) * total_threads + gid] = __float_as_uint(tmin);
+            spill[size_t(sp - lds_entries) * total_threads + gid] =
+                uint64_t(node) | (uint64_t(__float_as_uint(tmin)) << 32);
         }
         ++sp;
     }
 
-    __device__ void pop(uint32_t& node, float& tmin) {
+    __device__ __forceinline__ void pop(uint32_t& node, float& tmin) {
         --sp;
         if (sp < lds_entries) {
-            node = lds[(2 * sp) * block_size + lane];
-            tmin = __uint_as_float(lds[(2 * sp + 1) * block_size + lane]);
+            uint2 const e = lds[__umul24(sp, block_size) + lane];
+            node          = e.x;
+            tmin          = __uint_as_float(e.y);
         } else {
-            size_t const k = 2 * size_t(sp - lds_entries);
-            node           = spill[k * total_threads + gid];
-            tmin           = __uint_as_float(spill[(k + 1) * total_threads + gid]);
+            // an atomic load, so that the two branches' loads stay an LDS
+            // and a global one: merged, they become a flat load, which waits
+            // for both counters
+            uint64_t const e = __hip_atomic_load(&spill[size_t(sp - lds_entries) * total_threads + gid],
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SINGLETHREAD);
+            node             = uint32_t(e);
+            tmin             = __uint_as_float(uint32_t(e >> 32));
         }
     }
 };
@@ -597,7 +601,7 @@ __device__ __forceinline__ bool pop_next2(Stack2& stack, Ray const& ray, uint32_
         uint32_t e;
         float    tmin;
         stack.pop(e, tmin);
-        if (ray.max_t >= tmin) {
+        if (!(ray.max_t < tmin)) {
             unpack_node(e, data, meta);
             return true;
         }
@@ -605,35 +609,40 @@ __device__ __forceinline__ bool pop_next2(Stack2& stack, Ray const& ray, uint32_
     return false;
 }
 
-__device__ __forceinline__ bool inner_step2(float4 const* __restrict__ nodes, Stack2& stack,
-                                            Ray const& ray, uint32_t& data, uint32_t& meta) {
-    uint32_t const a = data;
-
-    float4 const alo = nodes[2 * size_t(a) + 0];
-    float4 const ahi = nodes[2 * size_t(a) + 1];
-    float4 const blo = nodes[2 * size_t(a) + 2];
-    float4 const bhi = nodes[2 * size_t(a) + 3];
-
-    float      ta, tb;
-    bool const ha = dev::slab_entry(alo, ahi, ray.o, ray.inv, ray.min_t, ray.max_t, ta);
-    bool const hb = dev::slab_entry(blo, bhi, ray.o, ray.inv, ray.min_t, ray.max_t, tb);
-
-    bool const flip = (ray.sign_bits >> node_axis(meta)) & 1u;
-    bool const hn   = flip ? hb : ha;
-    bool const hf   = flip ? ha : hb;
-
-    if (hn | hf) {
-        if (hn & hf) {
-            uint32_t const fd = __float_as_uint(flip ? alo.w : blo.w);
-            uint32_t const fm = __float_as_uint(flip ? ahi.w : bhi.w);
-            stack.push(pack_node(fd, fm), flip ? ta : tb);
-        }
-        bool const take_b = hn ? flip : !flip;
-        data              = __float_as_uint(take_b ? blo.w : alo.w);
-        meta              = __float_as_uint(take_b ? bhi.w : ahi.w);
+// Both children of a node tested: goes on with the near one (data, meta),
+// pushes the far one when both are hit; false when neither is.  The booleans
+// stay lane masks, so their logic runs on the scalar unit.
+__device__ __forceinline__ bool choose_child(Stack2& stack, bool ha, bool hb, float ta, float tb,
+                                             uint32_t da, uint32_t ma, uint32_t db, uint32_t mb,
+                                             uint32_t sign_bits, uint32_t& data, uint32_t& meta) {
+    bool const flip   = 0 != ((sign_bits >> node_axis(meta)) & 1u);
+    bool const both   = ha & hb;
+    bool const take_b = (both & flip) | (hb & !ha);
+    if (both) {
+        stack.push(pack_node(take_b ? da : db, take_b ? ma : mb), take_b ? ta : tb);
+    }
+    if (ha | hb) {
+        data = take_b ? db : da;
+        meta = take_b ? mb : ma;
         return true;
     }
-    return pop_next2(stack, ray, data, meta);
+    return false;
+}
+
+__device__ __forceinline__ bool inner_step2(float4 const* __restrict__ nodes, Stack2& stack,
+                                            Ray const& ray, uint32_t& data, uint32_t& meta) {
+    // 32-bit byte offsets: a packable tree has fewer than 2^22 nodes
+    char const* const pair = reinterpret_cast<char const*>(nodes) + (data << 5);
+    float4 const alo = *reinterpret_cast<float4 const*>(pair);
+    float4 const ahi = *reinterpret_cast<float4 const*>(pair + 16);
+    float4 const blo = *reinterpret_cast<float4 const*>(pair + 32);
+    float4 const bhi = *reinterpret_cast<float4 const*>(pair + 48);
+
+    float      ta, tb;
+    bool const ha = dev::slab_lean(alo, ahi, ray.o, ray.inv, ray.min_t, ray.max_t, ta);
+    bool const hb = dev::slab_lean(blo, bhi, ray.o, ray.inv, ray.min_t, ray.max_t, tb);
+    return choose_child(stack, ha, hb, ta, tb, __float_as_uint(alo.w), __float_as_uint(ahi.w),
+                        __float_as_uint(blo.w), __float_as_uint(bhi.w), ray.sign_bits, data, meta);
 }
 
 // A sibling pair from its 32-byte compressed record: each box coordinate is
@@ -661,31 +670,31 @@ __device__ __forceinline__ bool inner_step_q(Launch const& p, Stack2& stack, Ray
     float4 const bhi = make_float4(dequant(r1.x >> 16, sx, ox), dequant(r1.y & 0xFFFFu, sy, oy),
                                    dequant(r1.y >> 16, sz, oz), 0.f);
 
-    float      ta, tb;
-    bool const ha = dev::slab_entry(alo, ahi, ray.o, ray.inv, ray.min_t, ray.max_t, ta);
-    bool const hb = dev::slab_entry(blo, bhi, ray.o, ray.inv, ray.min_t, ray.max_t, tb);
-
-    bool const flip = (ray.sign_bits >> node_axis(meta)) & 1u;
-    bool const hn   = flip ? hb : ha;
-    bool const hf   = flip ? ha : hb;
-
-    if (hn | hf) {
-        if (hn & hf) {
-            stack.push(flip ? r1.z : r1.w, flip ? ta : tb);
-        }
-        bool const take_b = hn ? flip : !flip;
-        unpack_node(take_b ? r1.w : r1.z, data, meta);
-        return true;
-    }
-    return pop_next2(stack, ray, data, meta);
+    float          ta, tb;
+    bool const     ha = dev::slab_lean(alo, ahi, ray.o, ray.inv, ray.min_t, ray.max_t, ta);
+    bool const     hb = dev::slab_lean(blo, bhi, ray.o, ray.inv, ray.min_t, ray.max_t, tb);
+    uint32_t da, ma, db, mb;
+    unpack_node(r1.z, da, ma);
+    unpack_node(r1.w, db, mb);
+    return choose_child(stack, ha, hb, ta, tb, da, ma, db, mb, ray.sign_bits, data, meta);
 }
 
-// trace_refill<Any, true> with the two-word stack (trees of < 2^22 nodes and
-// slots); the same rays in the same order, the same results.  Quant: inner
-// nodes from the compressed pairs (kernel 4); a box of a pair holds the
-// original, so every node the exact boxes admit is visited, in the same
-// near / far order (the axis and the ray's sign decide it), and the
-// triangles are tested in the same relative order.
+// Persistent per-lane refill with the two-word stack (trees of < 2^22 nodes
+// and slots); the same rays visit the same nodes and triangles in the same
+// order as in trace_refill.  Quant: inner nodes from the compressed pairs
+// (kernel 4); a box of a pair holds the original, so every node the exact
+// boxes admit is visited, in the same near / far order (the axis and the
+// ray's sign decide it), and the triangles are tested in the same relative
+// order.
+//
+// Incoherent rays are bound by VALU issue at few active lanes (4.2 M bounce
+// rays over 1.41 M triangles: 1.28e9 wave instructions in 2.40 ms at 21.7 of
+// 64 lanes, when every lane was taken down to a leaf before any leaf was
+// tested).  So a turn of the loop is one step of one kind, the kind that most
+// of the wave's lanes wait for: a sibling pair for the lanes at inner nodes,
+// or one triangle for the lanes at leaves (1.84 ms; thresholds of 8 to 32
+// lanes before a change of kind: 2.06 to 1.92).  Pops of both kinds share one
+// loop, and the children's boxes go through slab_lean.
 template <bool Any, bool Quant>
 __global__ void trace_refill_packed(Launch p) {
     extern __shared__ uint32_t lds_stack[];
@@ -697,16 +706,17 @@ __global__ void trace_refill_packed(Launch p) {
     stack.init(lds_stack, p.spill, p.lds_entries, p.total_threads);
 
     uint32_t const lane     = threadIdx.x & 63;
-    uint64_t const lt_mask  = (uint64_t(1) << lane) - 1;
     uint32_t const num_rays = p.num_rays_dev ? *p.num_rays_dev : p.num_rays;
 
     Claims   claims;
-    claims.init();
     bool     active    = false;
     bool     exhausted = false;
-    uint32_t pool_next = 0;
-    uint32_t pool_end  = 0;
-    uint32_t r         = 0;
+    uint32_t pool_next;
+    uint32_t pool_end;
+    claims.init(__builtin_amdgcn_readfirstlane(stack.gid >> 6), p.total_threads >> 6, p.spread_waves,
+                num_rays, pool_next, pool_end);
+
+    uint32_t r = 0;
     Ray      ray;
     uint32_t data  = 0;
     uint32_t meta  = 0;
@@ -715,19 +725,17 @@ __global__ void trace_refill_packed(Launch p) {
     float    v     = 0.f;
 
     for (;;) {
-        uint64_t idle = __ballot(!active);
-        uint32_t const n_idle = uint32_t(__popcll(idle));
+        uint64_t live   = __ballot(active);
+        uint32_t n_idle = 64 - uint32_t(__popcll(live));
 
         if ((n_idle >= p.refill_lanes || 64 == n_idle) && !(exhausted && pool_next >= pool_end)) {
+            uint64_t idle = ~live;
             while (idle) {
                 if (pool_next >= pool_end) {
                     if (exhausted) {
                         break;
                     }
-                    uint32_t const leader =
-                        uint32_t(__ffsll(static_cast<unsigned long long>(idle))) - 1;
-                    if (!claims.next(p.counter, num_rays, p.claim_batch, lane, leader, pool_next,
-                                     pool_end)) {
+                    if (!claims.next(p.counter, num_rays, p.claim_batch, lane, pool_next, pool_end)) {
                         exhausted = true;
                         break;
                     }
@@ -736,7 +744,8 @@ __global__ void trace_refill_packed(Launch p) {
                 uint32_t const want  = uint32_t(__popcll(idle));
                 uint32_t const take  = avail < want ? avail : want;
                 bool const     mine  = (idle >> lane) & 1u;
-                uint32_t const rank  = uint32_t(__popcll(idle & lt_mask));
+                uint32_t const rank  = __builtin_amdgcn_mbcnt_hi(
+                    uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
                 if (mine && rank < take) {
                     r        = p.order ? p.order[pool_next + rank] : pool_next + rank;
                     ray      = load_ray(p.rays, r);
@@ -749,7 +758,7 @@ __global__ void trace_refill_packed(Launch p) {
                     float4 const rhi = nodes[1];
                     if (dev::slab(rlo, rhi, ray.o, ray.inv, ray.min_t, ray.max_t)) {
                         data   = __float_as_uint(rlo.w);
-                        meta   = __float_as_uint(rhi.w);
+                        meta   = __float_as_uint(rhi.w) & 0xFFFFu;
                         active = true;
                     } else {
                         write_result(p, r, Any, false, ray.max_t, Null, 0.f, 0.f);
@@ -758,38 +767,70 @@ __global__ void trace_refill_packed(Launch p) {
                 pool_next += take;
                 idle = __ballot(mine && rank >= take);
             }
+            live   = __ballot(active);
+            n_idle = 64 - uint32_t(__popcll(live));
         }
 
-        if (0 == __ballot(active)) {
+        if (0 == live) {
             if (exhausted && pool_next >= pool_end) {
                 break;
             }
             continue;
         }
 
-        while (__ballot(active && 0 == node_num(meta))) {
-            if (active && 0 == node_num(meta)) {
-                bool const more = Quant ? inner_step_q(p, stack, ray, data, meta)
-                                        : inner_step2(nodes, stack, ray, data, meta);
-                if (!more) {
+        // inner nodes, until most of the wave's lanes are at leaves or enough
+        // are idle (this loop leaves max_t, u, v and index alone)
+        bool const more    = !(exhausted && pool_next >= pool_end);
+        bool       at_leaf = active & (0 != node_num(meta));
+        uint32_t   n_live  = 64 - n_idle;
+        uint32_t   n_leaf  = uint32_t(__popcll(__ballot(at_leaf)));
+        while (2 * n_leaf <= n_live && !(more && 64 - n_live >= p.refill_lanes) && n_live) {
+            if (active & !at_leaf) {
+                bool const found = Quant ? inner_step_q(p, stack, ray, data, meta)
+                                         : inner_step2(nodes, stack, ray, data, meta);
+                if (!found && !pop_next2(stack, ray, data, meta)) {
                     write_result(p, r, Any, false, ray.max_t, index, u, v);
                     active = false;
                 }
             }
+            at_leaf = active & (0 != node_num(meta));
+            n_live  = uint32_t(__popcll(__ballot(active)));
+            n_leaf  = uint32_t(__popcll(__ballot(at_leaf)));
+        }
+        if (2 * n_leaf <= n_live) {
+            continue;  // idle lanes first
         }
 
-        if (active) {
-            uint32_t const num = node_num(meta);
-            bool           live;
-            bool           hit_p = false;
-            if (0 == num) {
-                live = inner_step2(nodes, stack, ray, data, meta);
-            } else {
-                uint32_t tests = 0;
-                hit_p          = leaf<Any>(tris, data, num, ray, index, u, v, tests);
-                live           = !hit_p && pop_next2(stack, ray, data, meta);
+        // one triangle per lane and turn, as long as half of the lanes that
+        // came with a leaf have triangles left
+        bool     pop   = false;
+        bool     hit_p = false;
+        uint32_t left;
+        do {
+            if (at_leaf) {
+                char const* const tri = reinterpret_cast<char const*>(tris) + __umul24(data, 48u);
+                float4 const      ta  = *reinterpret_cast<float4 const*>(tri);
+                float4 const      t1  = *reinterpret_cast<float4 const*>(tri + 16);
+                float4 const      t2  = *reinterpret_cast<float4 const*>(tri + 32);
+
+                float t, tu, tv;
+                if (dev::triangle({ta.x, ta.y, ta.z}, {t1.x, t1.y, t1.z}, {t2.x, t2.y, t2.z}, ray.o,
+                                  ray.d, ray.min_t, ray.max_t, t, tu, tv)) {
+                    hit_p     = true;
+                    ray.max_t = Any ? ray.max_t : t;
+                    u         = tu;
+                    v         = tv;
+                    index     = __float_as_uint(ta.w);
+                }
+                ++data;
+                meta -= 0x100u;
+                pop     = (Any && hit_p) || 0 == node_num(meta);
+                at_leaf = !pop;
             }
-            if (!live) {
+            left = uint32_t(__popcll(__ballot(at_leaf)));
+        } while (2 * left > n_leaf);
+        if (pop) {
+            if ((Any && hit_p) || !pop_next2(stack, ray, data, meta)) {
                 write_result(p, r, Any, hit_p, ray.max_t, index, u, v);
                 active = false;
             }
@@ -903,7 +944,7 @@ namespace {
 
 // The two-word stack holds node words of trees below 2^22 nodes and slots.
 bool packable(DeviceBvh const& bvh) {
-    return bvh.num_nodes < (1u << Packed_data_bits) && bvh.num_slots < (1u << Packed_data_bits);
+    return !bvh.nan_bounds && bvh.num_nodes < (1u << Packed_data_bits) && bvh.num_slots < (1u << Packed_data_bits);
 }
 
 // The compressed pairs of kernel 4 (made once per tree): a grid of 65 535
@@ -1110,6 +1151,7 @@ int32_t launch(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays, ui
     p.counter       = counter;
     p.refill_lanes  = res.refill_lanes;
     p.claim_batch   = res.claim_batch;
+    p.spread_waves  = res.spread_waves();
 
     if (counts) {
         if (any_hit) {

@@ -21,6 +21,8 @@ struct DeviceBvh {
     uint32_t num_slots     = 0;
     uint32_t num_triangles = 0;
     uint32_t max_depth     = 0;
+    bool     nan_bounds    = false;  // a vertex or node bound is not finite: only the traversals
+                                     // with the reference's NaN filters take the tree
 
     float  aabb_min[3] = {0.f, 0.f, 0.f};
     float  aabb_max[3] = {0.f, 0.f, 0.f};
@@ -68,8 +70,16 @@ struct TraceResources {
     size_t    sort_temp_bytes = 0;
     uint32_t  sort_capacity   = 0;
 
+    // Waves a small launch is spread over before its waves take 64 rays each
+    // (Claims): four per SIMD.  10 000 bounce rays over 340 k triangles ran
+    // 197, 190, 174 and 162 us at 0.5, 1, 2 and 4 waves per SIMD.
+    uint32_t spread_waves() const { return num_cus * 16; }
+
     uint32_t grid_blocks(uint32_t num_rays) const {
-        uint64_t const wanted   = (uint64_t(num_rays) + block_size - 1) / block_size;
+        uint64_t const want     = (uint64_t(num_rays) + spread_waves() - 1) / spread_waves();
+        uint64_t const chunk    = want < 64 ? (want ? want : 1) : 64;
+        uint64_t const waves    = (uint64_t(num_rays) + chunk - 1) / chunk;
+        uint64_t const wanted   = (waves * 64 + block_size - 1) / block_size;
         uint64_t const resident = uint64_t(num_cus) * blocks_per_cu;
         uint64_t const b        = wanted < resident ? wanted : resident;
         return uint32_t(b > 0 ? b : 1);
