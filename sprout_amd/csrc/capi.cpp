@@ -184,6 +184,7 @@ int32_t mi_release(void) {
     context->render_state.release();
     context->render_trace.release();
     context->light_scratch.release();
+    release_build_workspace();
     (void)hipFree(context->e_table);
     context->trace.release();
     delete context;

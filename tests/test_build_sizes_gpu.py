@@ -1,0 +1,66 @@
+"""The builder at the sizes where a node changes list (a wave's node of 64
+references, a workgroup's of 1024, more than one chunk) and at the settings
+that move those lines, node for node against the oracle."""
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+
+    from sprout_amd import bvh
+
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    bvh.init(0)
+    yield bvh
+    torch.cuda.synchronize()
+
+
+def soup(n, seed, long=0.1):
+    """n triangles, a tenth of them long ones that straddle many planes"""
+    rng = np.random.default_rng(seed)
+    c = rng.random((n, 1, 3))
+    size = np.where(rng.random((n, 1, 1)) < long, 0.6, 0.05)
+    pos = (c + size * (rng.random((n, 3, 3)) - 0.5)).astype(np.float32).reshape(-1, 3)
+    return pos, np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+
+
+def check(gpu, pos, idx, **settings):
+    import torch
+
+    tree = gpu.Builder_SAH(**settings).build(torch.from_numpy(pos).cuda(),
+                                             torch.from_numpy(idx.view(np.int32)).cuda())
+    nodes, slots = tree.download()
+    want = O.build(pos, idx, **settings)
+    assert O.nodes_equal(nodes.view(O.NODE_DTYPE), want.nodes)
+    assert np.array_equal(slots, want.slots)
+    return tree
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 63, 64, 65, 255, 1023, 1024, 1025, 2047, 2049, 4100, 30011])
+def test_sizes(gpu, n):
+    print(f"{n} triangles", flush=True)
+    check(gpu, *soup(n, n))
+
+
+@pytest.mark.parametrize("settings", [
+    dict(num_slices=64), dict(num_slices=1), dict(sweep_threshold=1024), dict(sweep_threshold=200),
+    dict(sweep_threshold=1), dict(max_primitives=1), dict(max_primitives=40),
+    dict(max_primitives=100, sweep_threshold=64), dict(sweep_threshold=3, max_primitives=8)])
+@pytest.mark.parametrize("n", [1500, 6000])
+def test_settings(gpu, settings, n):
+    print(f"{n} triangles, {settings}", flush=True)
+    check(gpu, *soup(n, 7), **settings)
+
+
+def test_more_references_than_a_quarter_over(gpu):
+    """a fifth of the triangles long: the levels outgrow the first two allocations"""
+    pos, idx = soup(20000, 9, long=0.2)
+    tree = check(gpu, pos, idx)
+    assert tree.info().num_slots > 2.6 * len(idx)
