@@ -37,20 +37,16 @@ struct Light_forest_out {
 };
 
 struct Light_forest_scratch {
-    uint32_t* mapping    = nullptr;
+    void*     recs       = nullptr;
+    uint32_t* owner      = nullptr;
+    void*     sides      = nullptr;
     void*     nodes      = nullptr;
     uint32_t* counters   = nullptr;
-    uint32_t* cand_node  = nullptr;
-    uint32_t* cand_k     = nullptr;
-    float*    cand_cost  = nullptr;
-    uint32_t* cand_start = nullptr;
-    uint32_t* cand_count = nullptr;
-    uint32_t* node_base  = nullptr;
-    uint32_t* light_root = nullptr;
-    uint32_t* cdf_base   = nullptr;
+    uint32_t* swap_left  = nullptr;
+    uint32_t* swap_right = nullptr;
     uint32_t* num_nodes  = nullptr;
     uint32_t* first      = nullptr;
-    uint32_t* counters_host = nullptr;  // pinned
+    uint32_t* host       = nullptr;  // page-locked
     uint32_t  light_capacity = 0;
     uint32_t  root_capacity  = 0;
 
@@ -58,7 +54,7 @@ struct Light_forest_scratch {
     void    release();
 };
 
-// Builds the forest on `stream` and waits for it (a level at a time).
+// Builds the forest on `stream` and waits for it.
 // MI_ERR_UNSPLITTABLE: a scene-tree node no candidate splits (the host
 // builder's median fallback); nothing else is wrong with the inputs.
 int32_t build_light_forest(Light_forest const& in, Light_forest_scratch& scratch,

@@ -87,27 +87,58 @@ __host__ __device__ inline bool same_bits(Cone const& a, Cone const& b) {
     return true;
 }
 
-// cone::merge, base/math/cone.inl:17-60
-__host__ __device__ inline Cone merge(Cone a, Cone b) {
-    if (1.f == a.v[0] && 1.f == a.v[1] && 1.f == a.v[2] && 1.f == a.v[3]) {
-        return b;
+__host__ __device__ inline bool empty(Cone const& a) {
+    return 1.f == a.v[0] && 1.f == a.v[1] && 1.f == a.v[2] && 1.f == a.v[3];
+}
+
+// A cone with the angle of its cosine (acos_r) and a sine of that angle.
+struct Wide {
+    Cone  cone;
+    float angle = 0.f;
+    float sine  = 0.f;
+};
+
+__host__ __device__ inline Wide wide(Cone const& c) {
+    return {c, acos_r(c.v[3]), sqrtf((1.f - c.v[3]) * (1.f + c.v[3]))};
+}
+
+// Whether cone b lies inside cone a for certain, so that merge gives a; told
+// from the cosines alone.  The axes' angle d fits d + b <= a where cos d >=
+// cos(a - b); as cosine is no steeper than 1, a cosine larger by Margin means
+// an angle smaller by at least Margin, more than the rounding of the float
+// angles and of this expression (under 2e-6 together).  With b = 0 (a flat
+// light's cone) or d = 0 the float angles order as their cosines do, without
+// a margin.  Cones nearer the edge, and NaNs, are left to the angles.
+__host__ __device__ inline bool inside(Wide const& a, Wide const& b) {
+    constexpr float Margin = 1e-5f;
+    float const     ca = a.cone.v[3], cb = b.cone.v[3];
+    float const     edge = 0.f == b.angle ? ca : ca * cb + a.sine * b.sine + Margin;
+    float const     x    = dot3(a.cone.v, b.cone.v);
+    return !empty(a.cone) && ((b.angle <= a.angle && smin(x, 1.f) >= smin(edge, 1.f)) ||
+                              same_bits(a.cone, b.cone));
+}
+
+// cone::merge, base/math/cone.inl:17-60, of cones whose angles are known
+__host__ __device__ inline Wide merge(Wide wa, Wide const& wb) {
+    if (empty(wa.cone)) {
+        return wb;
     }
-    if (same_bits(a, b)) {
-        return a;
+    if (inside(wa, wb)) {
+        return wa;
     }
-    float a_angle = acos_r(a.v[3]);
-    float b_angle = acos_r(b.v[3]);
+    Cone  a = wa.cone, b = wb.cone;
+    float a_angle = wa.angle;
+    float b_angle = wb.angle;
     if (b_angle > a_angle) {
-        Cone const t = a;
-        a            = b;
-        b            = t;
-        float const s = a_angle;
-        a_angle       = b_angle;
-        b_angle       = s;
+        a       = wb.cone;
+        b       = wa.cone;
+        a_angle = wb.angle;
+        b_angle = wa.angle;
+        wa      = wb;
     }
     float const d_angle = acos_r(smin(smax(dot3(a.v, b.v), -1.f), 1.f));
     if (smin(d_angle + b_angle, Pi) <= a_angle) {
-        return a;
+        return wa;
     }
     float const o_angle = (a_angle + d_angle + b_angle) / 2.f;
     // (the reference computes, and drops, a full-sphere cone when o_angle >= pi)
@@ -119,9 +150,8 @@ __host__ __device__ inline Cone merge(Cone a, Cone b) {
     if (!(cc > 0.f)) {
         // opposite axes: the reference normalizes a zero vector here and gets
         // a NaN cone; the cone that bounds both is the whole sphere
-        Cone r = a;
-        r.v[3] = -1.f;
-        return r;
+        a.v[3] = -1.f;
+        return wide(a);
     }
     float const cl = 1.f / sqrtf(cc);
     for (float& x : c) {
@@ -158,7 +188,14 @@ __host__ __device__ inline Cone merge(Cone a, Cone b) {
     r.v[1] = ax[1] * al;
     r.v[2] = ax[2] * al;
     r.v[3] = cos_r(o_angle);
-    return r;
+    return wide(r);
+}
+
+__host__ __device__ inline Cone merge(Cone const& a, Cone const& b) {
+    if (empty(a)) {
+        return b;
+    }
+    return merge(wide(a), wide(b)).cone;
 }
 
 __host__ __device__ inline float cone_cost(float cos) {
@@ -219,50 +256,69 @@ struct Candidate {
     // Split_candidate::evaluate over mapping[begin, end) of a node with
     // the given bounds and cone weight
     __host__ __device__ void evaluate(uint32_t begin, uint32_t end, uint32_t const* mapping,
-                                      Box const& bounds, float cone_weight, Light_set const& set) {
-        uint32_t n0 = 0, n1 = 0;
-        Box      b0, b1;
-        Cone     c0, c1;
-        bool     t0 = false, t1 = false;
-        float    p0 = 0.f, p1 = 0.f;
-        for (uint32_t i = begin; i < end; ++i) {
-            uint32_t const l     = mapping[i];
-            float const    power = set.powers[l];
-            if (0.f == power) {
-                continue;
-            }
-            float const* lo = set.lo + 3 * size_t(l);
-            float const* hi = set.hi + 3 * size_t(l);
-            if (behind(hi)) {
-                ++n0;
-                b0.merge(lo, hi);
-                c0 = merge(c0, set.cone(l));
-                t0 = t0 || set.two(l);
-                p0 += power;
-            } else {
-                ++n1;
-                b1.merge(lo, hi);
-                c1 = merge(c1, set.cone(l));
-                t1 = t1 || set.two(l);
-                p1 += power;
-            }
+                                      Box const& bounds, float cone_weight, Light_set const& set);
+};
+
+// One side of a split: its lights added in order, one by one.
+struct Side {
+    uint32_t n = 0;
+    Box      box;
+    Wide     cone;
+    float    power = 0.f;
+    bool     two   = false;
+};
+
+// Both sides of a split: Split_candidate::evaluate's fold over a node's lights
+// and the cost it comes to.
+struct Sides {
+    Side s0, s1;
+
+    __host__ __device__ static void add(Side& s, float light_power, float const* lo,
+                                        float const* hi, Wide const& light_cone, bool light_two) {
+        if (0.f == light_power) {
+            return;
         }
+        ++s.n;
+        s.box.merge(lo, hi);
+        s.cone = merge(s.cone, light_cone);
+        s.two  = s.two || light_two;
+        s.power += light_power;
+    }
+
+    // the candidate's sides and cost, for a node of len lights
+    __host__ __device__ void finish(uint32_t len, Box const& bounds, float cone_weight,
+                                    Candidate& c) const {
         float const e0  = bounds.extent(0), e1 = bounds.extent(1), e2 = bounds.extent(2);
-        float const reg = smax(smax(e0, e1), e2) / bounds.extent(axis);
+        float const reg = smax(smax(e0, e1), e2) / bounds.extent(c.axis);
         float const sa  = bounds.surface_area();
-        box0 = b0, box1 = b1, cone0 = c0, cone1 = c1, power0 = p0, power1 = p1, two0 = t0, two1 = t1;
-        if (0 == n0 || 0 == n1) {
-            cost      = 2.f * reg * (p0 + p1) * (4.f * Pi) * sa * float(end - begin);
-            exhausted = true;
+        c.box0 = s0.box, c.cone0 = s0.cone.cone, c.power0 = s0.power, c.two0 = s0.two;
+        c.box1 = s1.box, c.cone1 = s1.cone.cone, c.power1 = s1.power, c.two1 = s1.two;
+        if (0 == s0.n || 0 == s1.n) {
+            c.cost      = 2.f * reg * (s0.power + s1.power) * (4.f * Pi) * sa * float(len);
+            c.exhausted = true;
         } else {
-            float const wa = cone_cost(c0.v[3]) * (t0 ? 2.f : 1.f);
-            float const wb = cone_cost(c1.v[3]) * (t1 ? 2.f : 1.f);
-            cost = reg * (((p0 * wa * b0.surface_area()) + (p1 * wb * b1.surface_area())) /
-                          (sa * cone_weight));
-            exhausted = false;
+            float const wa = cone_cost(s0.cone.cone.v[3]) * (s0.two ? 2.f : 1.f);
+            float const wb = cone_cost(s1.cone.cone.v[3]) * (s1.two ? 2.f : 1.f);
+            c.cost         = reg * (((s0.power * wa * s0.box.surface_area()) +
+                             (s1.power * wb * s1.box.surface_area())) /
+                            (sa * cone_weight));
+            c.exhausted = false;
         }
     }
 };
+
+__host__ __device__ inline void Candidate::evaluate(uint32_t begin, uint32_t end,
+                                                    uint32_t const* mapping, Box const& bounds,
+                                                    float cone_weight, Light_set const& set) {
+    Sides s;
+    for (uint32_t i = begin; i < end; ++i) {
+        uint32_t const l  = mapping[i];
+        float const*   hi = set.hi + 3 * size_t(l);
+        Sides::add(behind(hi) ? s.s0 : s.s1, set.powers[l], set.lo + 3 * size_t(l), hi,
+                   wide(set.cone(l)), set.two(l));
+    }
+    s.finish(end - begin, bounds, cone_weight, *this);
+}
 
 // The number of split candidates of a node of len lights (sweep below the
 // threshold: three per light; else the 16-slice grid of
