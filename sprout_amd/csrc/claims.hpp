@@ -27,6 +27,19 @@ namespace mi {
 // sees runs of 4 Claim_run claims.
 inline constexpr uint32_t Claim_run = 8;
 
+// Rays of a wave's slice.
+__host__ __device__ inline uint32_t claim_chunk(uint32_t num_rays, uint32_t waves, uint32_t spread) {
+    uint32_t const over = waves < spread ? waves : spread;
+    uint32_t const want = num_rays / over + (num_rays % over ? 1u : 0u);
+    return want < 64u ? want : 64u;
+}
+
+// Whether rays are left over past the slices: only then does a launch touch
+// its counters.
+inline bool claims_rays(uint32_t num_rays, uint32_t waves, uint32_t spread) {
+    return uint64_t(waves) * claim_chunk(num_rays, waves, spread) < num_rays;
+}
+
 struct Claims {
     uint32_t part;   // wave-uniform: the part claimed from
     uint32_t parts;  // all parts (at most the launch's waves, so each has a wave)
@@ -36,9 +49,7 @@ struct Claims {
     // the launch's, spread the number of waves a small launch fills first.
     __device__ void init(uint32_t wave, uint32_t waves, uint32_t spread, uint32_t num_rays,
                          uint32_t& begin, uint32_t& end) {
-        uint32_t const over  = waves < spread ? waves : spread;
-        uint32_t const want  = num_rays / over + (num_rays % over ? 1u : 0u);
-        uint32_t const chunk = want < 64u ? want : 64u;
+        uint32_t const chunk = claim_chunk(num_rays, waves, spread);
         uint64_t const all   = uint64_t(waves) * chunk;
         fixed                = all < num_rays ? uint32_t(all) : num_rays;
         uint64_t const lo    = uint64_t(wave) * chunk;

@@ -731,7 +731,8 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
 }
 
 int32_t trace_instances_launch(Tlas const& t, uint32_t num_cus, mi_ray const* rays, uint32_t n,
-                               uint32_t const* n_dev, void* out, bool any_hit, hipStream_t stream) {
+                               uint32_t const* n_dev, void* out, bool any_hit, hipStream_t stream,
+                               uint32_t* claims) {
     if (0 == n) {
         return MI_OK;
     }
@@ -743,13 +744,16 @@ int32_t trace_instances_launch(Tlas const& t, uint32_t num_cus, mi_ray const* ra
         uint64_t const chunk  = std::min<uint64_t>(want, 64);
         uint64_t const wanted = (uint64_t(n) + chunk - 1) / chunk;
         uint32_t const blocks = uint32_t(std::min<uint64_t>(wanted, t.spill_total / Block2));
-        hipLaunchKernelGGL(reset_claims, dim3(1), dim3(64), 0, stream, t.claims);
+        uint32_t* const counters = claims ? claims : t.claims;
+        if (!claims && (n_dev || claims_rays(n, blocks * (Block2 / 64), spread))) {
+            hipLaunchKernelGGL(reset_claims, dim3(1), dim3(64), 0, stream, counters);
+        }
         if (any_hit) {
             hipLaunchKernelGGL(trace_instances_refill<true>, dim3(blocks), dim3(Block2), 0, stream, v,
-                               t.spill, t.spill_total, t.claims, rays, n, n_dev, spread, out);
+                               t.spill, t.spill_total, counters, rays, n, n_dev, spread, out);
         } else {
             hipLaunchKernelGGL(trace_instances_refill<false>, dim3(blocks), dim3(Block2), 0, stream, v,
-                               t.spill, t.spill_total, t.claims, rays, n, n_dev, spread, out);
+                               t.spill, t.spill_total, counters, rays, n, n_dev, spread, out);
         }
         if (hipError_t const e = hipGetLastError(); e) {
             return fail(MI_ERR_HIP, "instance trace: %s", hipGetErrorString(e));

@@ -95,8 +95,11 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
 
 // Closest (out: mi_instance_hit per ray, pad[0] = the mesh tree's slot) or
 // any hit (out: uint32 per ray).  n_dev (optional): a ray count in device
-// memory, at most n (capturable).
+// memory, at most n (capturable).  claims (optional): ray claim counters
+// (Counter_words) of the launch's own, zero when it starts; else the tree's,
+// which the call clears.
 int32_t trace_instances_launch(Tlas const& t, uint32_t num_cus, mi_ray const* rays, uint32_t n,
-                               uint32_t const* n_dev, void* out, bool any_hit, hipStream_t stream);
+                               uint32_t const* n_dev, void* out, bool any_hit, hipStream_t stream,
+                               uint32_t* claims = nullptr);
 
 }  // namespace mi

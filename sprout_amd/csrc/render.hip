@@ -77,9 +77,23 @@ constexpr uint32_t C_base       = 3 * Counter_line;  // first sample index of th
 constexpr uint32_t C_records    = 4 * Counter_line;  // training samples recorded in the current wave
 constexpr uint32_t C_totals     = 5 * Counter_line;  // two uint64: extension and shadow rays traced,
                                                      // then one uint64: guiding records trained on
-constexpr uint32_t C_done       = 6 * Counter_line;  // regenerating: paths that ended this bounce
-constexpr uint32_t C_next       = 7 * Counter_line;  // regenerating: the next sample of the batch to start
-constexpr uint32_t Num_counters = 8 * Counter_line;
+constexpr uint32_t C_next       = 6 * Counter_line;  // regenerating: the next sample of the batch to start
+constexpr uint32_t C_resolve    = 7 * Counter_line;  // the vertices whose shadow rays are resolved
+constexpr uint32_t C_done0      = 8 * Counter_line;  // regenerating: paths that ended this bounce, by queue
+constexpr uint32_t C_claims     = 10 * Counter_line; // the traversals' ray claims
+constexpr uint32_t Num_counters = C_claims + Counter_words;
+
+// No kernel of a bounce exists to clear or add up counters (four of one
+// thread each, 4.7 us apiece, were 0.17 ms of a 1.9 ms frame of nine
+// bounces): raygen clears them, and each is cleared again by the first thread
+// of a kernel that runs when the last reader is done and the next writer has
+// not begun:
+//   claims          shade (after the closest hits), shadow_resolve (after the
+//                   shadow rays), for the traversal that follows
+//   queue in_q      nee, which adds it to the totals and leaves its length in
+//                   C_resolve; the next bounce fills it
+//   shadow queue    shadow_resolve; nee adds it to the totals
+//   done, in_q ^ 1  nee; regenerate read it the bounce before
 
 // rnd::Generator, base/random/generator.inl:16-49
 struct Rng {
@@ -594,10 +608,6 @@ __global__ void set_base(uint32_t* counters, uint32_t first_sample) {
     }
 }
 
-__global__ void advance_base(uint32_t* counters, uint32_t samples) {
-    counters[C_base] += samples;
-}
-
 // Starts sample k of the frame batch (plane k / num_pixels, pixel k %
 // num_pixels of the camera grid) in path slot `slot`: the camera sample and
 // the path state; returns the camera ray.
@@ -673,6 +683,13 @@ __device__ mi_ray start_path(Wave const& w, uint32_t k, uint32_t slot) {
     return r;
 }
 
+// The traversal that follows hands out its rays from the start.
+__device__ __forceinline__ void clear_claims(Wave const& w) {
+    if (0 == blockIdx.x && threadIdx.x < Claim_parts) {
+        w.counters[C_claims + threadIdx.x * Claim_stride] = 0;
+    }
+}
+
 // The first rays of a wave (or of a regenerating batch): sample p in slot p
 // for the first min(num_paths, batch_samples) slots.
 __global__ void __launch_bounds__(256) raygen(Wave w) {
@@ -682,27 +699,15 @@ __global__ void __launch_bounds__(256) raygen(Wave w) {
         w.rays[0][p]     = start_path(w, p, p);
         w.ray_path[0][p] = p;
     }
+    clear_claims(w);
     if (0 == p) {
         w.counters[C_queue0]                = live;
         w.counters[C_queue0 + Counter_line] = 0;
         w.counters[C_shadow]                = 0;
-        w.counters[C_done]                  = 0;
+        w.counters[C_done0]                 = 0;
+        w.counters[C_done0 + Counter_line]  = 0;
         w.counters[C_next]                  = live;  // the next sample to start
     }
-}
-
-// Clears the queue the next shade fills and the shadow queue.
-__global__ void reset_queues(uint32_t* counters, uint32_t out_q) {
-    counters[C_queue0 + Counter_line * out_q] = 0;
-    counters[C_shadow]                        = 0;
-    counters[C_done]                          = 0;
-}
-
-// Ray totals for the statistics: the queue just traced and the shadow queue.
-__global__ void tally(uint32_t* counters, uint32_t in_q) {
-    uint64_t* totals = reinterpret_cast<uint64_t*>(counters + C_totals);
-    totals[0] += counters[C_queue0 + Counter_line * in_q];
-    totals[1] += counters[C_shadow];
 }
 
 // The collision coefficients per unit density at a path's four wavelengths.
@@ -831,6 +836,7 @@ __device__ __forceinline__ void shade_queue(Wave const& w, uint32_t in_q) {
     uint32_t const count  = w.counters[C_queue0 + Counter_line * in_q];
     uint32_t const out_q  = in_q ^ 1;
     uint32_t const stride = gridDim.x * blockDim.x;
+    clear_claims(w);
 
     // block-uniform trip count: every lane reaches the wave-wide queue appends
     for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
@@ -1233,7 +1239,7 @@ __device__ __forceinline__ void shade_queue(Wave const& w, uint32_t in_q) {
             // the path ends here: its slot goes to the next sample once the
             // vertex's shadow rays are resolved
             bool const     ended = i < count && !spawn;
-            uint32_t const d     = block_queue_range(ended ? 1u : 0u, &w.counters[C_done]);
+            uint32_t const d     = block_queue_range(ended ? 1u : 0u, &w.counters[C_done0 + Counter_line * in_q]);
             if (ended) {
                 w.done[d] = p;
             }
@@ -1266,7 +1272,7 @@ __global__ void __launch_bounds__(256) shade_guided(Wave w, uint32_t in_q) {
 // queue the next bounce traces.  One atomic per block for the samples and
 // one for the queue.
 __global__ void __launch_bounds__(256) regenerate(Wave w, uint32_t out_q) {
-    uint32_t const count  = w.counters[C_done];
+    uint32_t const count  = w.counters[C_done0 + Counter_line * (out_q ^ 1)];
     uint32_t const stride = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {  // block-uniform
         uint32_t const i    = base + threadIdx.x;
@@ -1302,6 +1308,9 @@ __global__ void __launch_bounds__(256) resolve_samples(Wave w, uint32_t planes, 
     if (pixel >= w.num_pixels) {
         return;
     }
+    if (0 == pixel) {
+        w.counters[C_base] += planes;  // the next wave's samples
+    }
     double a[3] = {accum[3 * size_t(pixel) + 0], accum[3 * size_t(pixel) + 1],
                    accum[3 * size_t(pixel) + 2]};
     for (uint32_t k0 = 0; k0 < planes; k0 += spw) {
@@ -1331,9 +1340,18 @@ __global__ void __launch_bounds__(256) resolve_samples(Wave w, uint32_t planes, 
 // Spectral: the contribution per wavelength (the fourth in shadow_c4), the
 // light's emission and the reflection upsampled to the path's wavelengths.
 template <bool Spectral>
-__device__ __forceinline__ void nee_queue(Wave const& w) {
+__device__ __forceinline__ void nee_queue(Wave const& w, uint32_t in_q) {
     uint32_t const count  = w.counters[C_shadow];
     uint32_t const stride = gridDim.x * blockDim.x;
+    if (0 == blockIdx.x && 0 == threadIdx.x) {
+        uint64_t* const totals = reinterpret_cast<uint64_t*>(w.counters + C_totals);
+        uint32_t const  rays   = w.counters[C_queue0 + Counter_line * in_q];
+        totals[0] += rays;
+        totals[1] += count;
+        w.counters[C_resolve]                             = rays;
+        w.counters[C_queue0 + Counter_line * in_q]        = 0;
+        w.counters[C_done0 + Counter_line * (in_q ^ 1)]   = 0;
+    }
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < count; j += stride) {
         Pick_slot const  pick = w.picks[j];
         Nee_vertex const v    = w.nee[pick.vertex];
@@ -1449,12 +1467,12 @@ __device__ __forceinline__ void nee_queue(Wave const& w) {
     }
 }
 
-__global__ void __launch_bounds__(256) nee(Wave w) {
-    nee_queue<false>(w);
+__global__ void __launch_bounds__(256) nee(Wave w, uint32_t in_q) {
+    nee_queue<false>(w, in_q);
 }
 
-__global__ void __launch_bounds__(256) nee_spectral(Wave w) {
-    nee_queue<true>(w);
+__global__ void __launch_bounds__(256) nee_spectral(Wave w, uint32_t in_q) {
+    nee_queue<true>(w, in_q);
 }
 
 // Adds the unoccluded light contributions of every vertex shaded this
@@ -1467,8 +1485,12 @@ __global__ void __launch_bounds__(256) nee_spectral(Wave w) {
 template <bool Spectral>
 __device__ __forceinline__ void shadow_resolve_queue(Wave const& w, uint32_t in_q) {
     constexpr int  NC     = Spectral ? 4 : 3;
-    uint32_t const count  = w.counters[C_queue0 + Counter_line * in_q];
+    uint32_t const count  = w.counters[C_resolve];
     uint32_t const stride = gridDim.x * blockDim.x;
+    clear_claims(w);
+    if (0 == blockIdx.x && 0 == threadIdx.x) {
+        w.counters[C_shadow] = 0;
+    }
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride) {
         uint2 const range = w.shadow_range[i];
         if (0 == range.y) {
@@ -1669,6 +1691,9 @@ __global__ void __launch_bounds__(256) resolve(Wave w, uint32_t planes, double* 
     if (pixel >= w.num_pixels) {
         return;
     }
+    if (0 == pixel) {
+        w.counters[C_base] += planes;  // the next wave's samples
+    }
     double s[3] = {0.0, 0.0, 0.0};
     for (uint32_t k = 0; k < planes; ++k) {
         Path const& p = w.paths[size_t(k) * w.num_pixels + pixel];
@@ -1716,6 +1741,9 @@ __global__ void __launch_bounds__(256) resolve_filtered(Wave w, uint32_t planes,
     uint32_t const pixel = blockIdx.x * blockDim.x + threadIdx.x;
     if (pixel >= uint32_t(w.width) * w.height) {
         return;
+    }
+    if (0 == pixel) {
+        w.counters[C_base] += planes;  // the next wave's samples
     }
     Sensor_filter const& f  = w.filter;
     int32_t const        bd = w.border;
@@ -3609,22 +3637,24 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
 
     // traversals with their ray counts on the device: the scene's tree, or
     // the top-level tree over instances
+    uint32_t* const claims = state.counters + C_claims;
     auto trace_closest = [&](mi_ray const* rays, uint32_t const* count) -> int32_t {
         if (scene.instanced) {
             return trace_instances_launch(scene.tlas, trace.num_cus, rays, num_paths, count,
-                                          state.inst_hits, false, s);
+                                          state.inst_hits, false, s, claims);
         }
         return launch_trace_device_count(scene.bvh, trace, rays, count, num_paths, state.hits,
-                                         false, s);
+                                         false, s, claims);
     };
     auto trace_any = [&]() -> int32_t {
         if (scene.instanced) {
             return trace_instances_launch(scene.tlas, trace.num_cus, state.shadow_rays, num_shadow,
-                                          &state.counters[C_shadow], state.occluded, true, s);
+                                          &state.counters[C_shadow], state.occluded, true, s,
+                                          claims);
         }
         return launch_trace_device_count(scene.bvh, trace, state.shadow_rays,
                                          &state.counters[C_shadow], num_shadow, state.occluded,
-                                         true, s);
+                                         true, s, claims);
     };
 
     // one wave: every kernel reads its counts and sample base on the device
@@ -3643,7 +3673,6 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
                 hipLaunchKernelGGL(spectral ? medium_track_spectral : medium_track,
                                    dim3(grid_path), dim3(256), 0, s, w, q);
             }
-            hipLaunchKernelGGL(reset_queues, dim3(1), dim3(1), 0, s, state.counters, q ^ 1);
             if (guided && d < guide_depth) {
                 hipLaunchKernelGGL(guide_inputs, dim3(grid_path), dim3(256), 0, s, w, q);
                 if (int32_t const st = guide_forward_device_count(
@@ -3662,8 +3691,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
                 hipLaunchKernelGGL(spectral ? shade_spectral : shade, dim3(grid_path), dim3(256),
                                    0, s, w, q);
             }
-            hipLaunchKernelGGL(spectral ? nee_spectral : nee, dim3(grid_shadow), dim3(256), 0, s, w);
-            hipLaunchKernelGGL(tally, dim3(1), dim3(1), 0, s, state.counters, q);
+            hipLaunchKernelGGL(spectral ? nee_spectral : nee, dim3(grid_shadow), dim3(256), 0, s, w, q);
             if (int32_t const st = trace_any(); st) {
                 return st;
             }
@@ -3677,7 +3705,6 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
         } else {
             hipLaunchKernelGGL(resolve, dim3(blocks(num_pixels, 256)), dim3(256), 0, s, w, spw, accum);
         }
-        hipLaunchKernelGGL(advance_base, dim3(1), dim3(1), 0, s, state.counters, spw);
         return MI_OK;
     };
 
@@ -3712,10 +3739,8 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             hipLaunchKernelGGL(spectral ? medium_track_spectral : medium_track, dim3(grid_path),
                                dim3(256), 0, s, w, q);
         }
-        hipLaunchKernelGGL(reset_queues, dim3(1), dim3(1), 0, s, state.counters, q ^ 1);
         hipLaunchKernelGGL(spectral ? shade_spectral : shade, dim3(grid_path), dim3(256), 0, s, w, q);
-        hipLaunchKernelGGL(spectral ? nee_spectral : nee, dim3(grid_shadow), dim3(256), 0, s, w);
-        hipLaunchKernelGGL(tally, dim3(1), dim3(1), 0, s, state.counters, q);
+        hipLaunchKernelGGL(spectral ? nee_spectral : nee, dim3(grid_shadow), dim3(256), 0, s, w, q);
         if (int32_t const st = trace_any(); st) {
             return st;
         }
@@ -3837,7 +3862,6 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             }
             hipLaunchKernelGGL(resolve_samples, dim3(blocks(num_pixels, 256)), dim3(256), 0, s, w,
                                batch_planes, spw, accum);
-            hipLaunchKernelGGL(advance_base, dim3(1), dim3(1), 0, s, state.counters, batch_planes);
         }
     } else if (set.flags & MI_RENDER_NO_GRAPH) {
         for (uint32_t wave = 0; wave < waves; ++wave) {

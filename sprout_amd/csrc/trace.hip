@@ -1030,9 +1030,10 @@ struct Fixed_scratch {
 // num_rays is only its upper bound (it sizes the grid and the stack spill).
 // fixed set: the launch allocates nothing and uses fixed's counter and spill
 // area, with as many workgroups (at most the usual grid) as the area holds.
+// claims set: ray claim counters that are zero already.
 int32_t launch(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays, uint32_t num_rays,
                uint32_t const* num_rays_dev, void* out, uint32_t* counts, bool any_hit,
-               hipStream_t stream, Fixed_scratch const* fixed = nullptr) {
+               hipStream_t stream, Fixed_scratch const* fixed = nullptr, uint32_t* claims = nullptr) {
     if (0 == num_rays) {
         return MI_OK;
     }
@@ -1072,9 +1073,16 @@ int32_t launch(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays, ui
             return st;
         }
         spill   = res.spill;
-        counter = res.counter;
+        counter = claims ? claims : res.counter;
     }
     uint32_t const threads = blocks * block;
+    // a launch whose waves' own slices hold all rays claims none
+    bool const claiming = num_rays_dev || claims_rays(num_rays, threads >> 6, res.spread_waves());
+    auto const reset    = [&] {
+        if (!claims && claiming) {
+            hipLaunchKernelGGL(reset_counter, dim3(1), dim3(64), 0, stream, counter);
+        }
+    };
 
     size_t const lds_bytes = size_t(sl.words) * lds_entries * block * sizeof(uint32_t);
 
@@ -1160,13 +1168,13 @@ int32_t launch(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays, ui
             hipLaunchKernelGGL(trace_reference<false>, dim3(blocks), dim3(block), lds_bytes, stream, p);
         }
     } else if (packed) {
-        hipLaunchKernelGGL(reset_counter, dim3(1), dim3(64), 0, stream, counter);
+        reset();
         using Kernel = void (*)(Launch);
         Kernel const kern = any_hit ? (quant ? trace_refill_packed<true, true> : trace_refill_packed<true, false>)
                                     : (quant ? trace_refill_packed<false, true> : trace_refill_packed<false, false>);
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), lds_bytes, stream, p);
     } else if (res.kernel != 1 || num_rays_dev) {
-        hipLaunchKernelGGL(reset_counter, dim3(1), dim3(64), 0, stream, counter);
+        reset();
         using Kernel    = void (*)(Launch);
         bool const ww   = 2 <= res.kernel;
         Kernel     kern = any_hit ? (ww ? trace_refill<true, true> : trace_refill<true, false>)
@@ -1212,8 +1220,8 @@ int32_t launch_trace(DeviceBvh const& bvh, TraceResources& res, mi_ray const* ra
 
 int32_t launch_trace_device_count(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays,
                                   uint32_t const* num_rays, uint32_t max_rays, void* out,
-                                  bool any_hit, hipStream_t stream) {
-    return launch(bvh, res, rays, max_rays, num_rays, out, nullptr, any_hit, stream);
+                                  bool any_hit, hipStream_t stream, uint32_t* claims) {
+    return launch(bvh, res, rays, max_rays, num_rays, out, nullptr, any_hit, stream, nullptr, claims);
 }
 
 // ---- closest hit without allocation ----

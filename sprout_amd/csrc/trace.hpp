@@ -112,10 +112,11 @@ int32_t prepare_trace(DeviceBvh const& bvh, TraceResources& res, uint32_t max_ra
 
 // Same traversal over a ray count that lives in device memory (written by an
 // earlier kernel on the stream); max_rays bounds it.  Capturable: it records
-// kernels only.
+// one kernel only.  claims: the launch's ray claim counters (Counter_words),
+// zero when it starts.
 int32_t launch_trace_device_count(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays,
                                   uint32_t const* num_rays, uint32_t max_rays, void* out,
-                                  bool any_hit, hipStream_t stream);
+                                  bool any_hit, hipStream_t stream, uint32_t* claims);
 
 // Sets up the fixed scratch of launch_trace_noalloc on `device`, which must
 // be the current device (once per device; later calls return at once).
