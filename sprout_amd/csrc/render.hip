@@ -67,6 +67,9 @@ using dev::v3;
 
 constexpr float Ray_max_t = 3.40282347e+38f;
 
+// Waves of one call from which on a new wave description is captured at once.
+constexpr uint32_t Capture_waves = 16;
+
 // Counter words of RenderState::counters, each on its own 256-byte line:
 // atomics on one line serialize (about 12 ns each), so the two queues the
 // shading kernel appends to must not share one.
@@ -3878,6 +3881,12 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
         // The wave's graph is kept between calls: everything its kernels take
         // (the wave description, buffers, launch shapes, training settings)
         // forms the key, and an equal key replays the cached graph.
+        // Capturing and instantiating a wave costs 0.1 ms (9 bounces, 47
+        // kernels) that the first wave waits for, and a replayed wave runs
+        // 1 to 2 % faster than a launched one, so a key is captured when it
+        // comes a second time running, or for many waves: with the camera
+        // moved each frame, frames of 1 / 4 / 16 waves of 97x61 took 0.60 /
+        // 1.95 / 7.38 ms captured and 0.49 / 1.88 / 7.43 ms launched.
         std::vector<uint8_t> key(sizeof(Wave));
         std::memcpy(key.data(), &w, sizeof(Wave));
         auto put = [&key](auto const& v) {
@@ -3908,7 +3917,21 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             put(records);
             put(state.shuf_x);
         }
-        if (!state.graph || key != state.graph_key) {
+        bool const cached  = state.graph && key == state.graph_key;
+        bool const capture = !cached && (key == state.last_key || waves >= Capture_waves);
+        state.last_key     = key;
+        if (!cached && !capture) {
+            for (uint32_t wave = 0; wave < waves; ++wave) {
+                if (int32_t const st = enqueue_wave(); st) {
+                    return st;
+                }
+                if (training) {
+                    if (int32_t const st = enqueue_training(); st) {
+                        return st;
+                    }
+                }
+            }
+        } else if (capture) {
             if (state.graph) {
                 (void)hipStreamSynchronize(s);  // its earlier launches may still run
                 (void)hipGraphExecDestroy(state.graph);
@@ -3942,7 +3965,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             }
             state.graph_key = std::move(key);
         }
-        for (uint32_t wave = 0; wave < waves && !e; ++wave) {
+        for (uint32_t wave = 0; wave < waves && !e && (cached || capture); ++wave) {
             e = hipGraphLaunch(state.graph, s);
         }
         if (e) {

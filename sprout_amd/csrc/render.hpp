@@ -212,6 +212,7 @@ struct RenderState {
     hipEvent_t   end         = nullptr;
     hipGraphExec_t       graph = nullptr;  // the last wave's graph, replayed while its key holds
     std::vector<uint8_t> graph_key;
+    std::vector<uint8_t> last_key;         // the last wave's, captured or not
     // guiding
     uint32_t  guide_capacity  = 0;
     float*    guide_x         = nullptr;  // network inputs per queue entry
