@@ -52,6 +52,8 @@ namespace dev {
 inline constexpr int32_t  Log2_cell_dim = 5;
 inline constexpr int32_t  Cell_dim      = 1 << Log2_cell_dim;
 inline constexpr uint32_t Grid_empty    = 0x7FFFFFFFu;
+inline constexpr int32_t  Log2_block_dim = 3;     // the smallest leaves
+inline constexpr uint8_t  Leaf_empty     = 0x80;
 inline constexpr float    Min_mt        = 1e-10f;
 inline constexpr float    Abort_epsilon = 7.5e-4f;
 inline constexpr uint32_t SR_low        = 16;
@@ -62,8 +64,8 @@ struct Medium_view {
     int32_t          dims[3];
     float            inv_dims[3];
     uint32_t         num_cells[3];
-    uint32_t const*  nodes;
-    Medium_cm const* data;
+    uint8_t const*   levels;  // per block of Block_dim^3 voxels: level of its leaf, | Leaf_empty
+    Medium_cm const* leaves;  // per block: its leaf's coefficients
     float            box_lo[3];
     float            iext[3];  // 1 / extent of the box
     float            cc_a[3];
@@ -152,7 +154,9 @@ __device__ inline bool intersect_inside(V3 lo, V3 hi, Tray const& r, float& hit_
     return max_out >= r.min_t && r.min_t >= min_out && r.max_t >= min_out && max_out >= min_out;
 }
 
-// Gridtree::intersect: clips r.max_t to the leaf cell around r.point(min_t)
+// Gridtree::intersect: clips r.max_t to the leaf cell around r.point(min_t).
+// The tree's leaves are laid out per block of its smallest leaf size, so a
+// cell is one load away instead of a chain of up to four.
 __device__ inline bool gridtree_intersect(Medium_view const& m, Tray& r, Medium_cm& cm) {
     V3 const      p  = r.point(r.min_t);
     int32_t const cx = int32_t(float(m.dims[0]) * p.x);
@@ -165,27 +169,15 @@ __device__ inline bool gridtree_intersect(Medium_view const& m, Tray& r, Medium_
         uint32_t(vz) >= m.num_cells[2]) {
         return false;
     }
-    uint32_t index = (uint32_t(vz) * m.num_cells[1] + uint32_t(vy)) * m.num_cells[0] + uint32_t(vx);
-    int32_t  b0[3] = {vx << Log2_cell_dim, vy << Log2_cell_dim, vz << Log2_cell_dim};
-    int32_t  b1[3] = {b0[0] + Cell_dim, b0[1] + Cell_dim, b0[2] + Cell_dim};
-    int32_t const c[3] = {cx, cy, cz};
-    for (;;) {
-        uint32_t const node = m.nodes[index];
-        if (0 == (node & 1u)) {
-            break;
-        }
-        index = node >> 1;
-        for (int k = 0; k < 3; ++k) {
-            int32_t const half   = (b1[k] - b0[k]) >> 1;
-            int32_t const center = b0[k] + half;
-            if (c[k] < center) {
-                b1[k] = center;
-            } else {
-                b0[k] = center;
-                index += 1u << k;
-            }
-        }
-    }
+    uint32_t const bx    = m.num_cells[0] << (Log2_cell_dim - Log2_block_dim);
+    uint32_t const by    = m.num_cells[1] << (Log2_cell_dim - Log2_block_dim);
+    size_t const   block = (size_t(cz >> Log2_block_dim) * by + uint32_t(cy >> Log2_block_dim)) * bx +
+                         uint32_t(cx >> Log2_block_dim);
+    uint32_t const level = m.levels[block];
+    Medium_cm const leaf = m.leaves[block];
+    int32_t const  size  = Cell_dim >> (level & 3u);
+    int32_t const  b0[3] = {cx & -size, cy & -size, cz & -size};
+    int32_t const  b1[3] = {b0[0] + size, b0[1] + size, b0[2] + size};
     V3 const lo = v3(float(b0[0]) * m.inv_dims[0], float(b0[1]) * m.inv_dims[1], float(b0[2]) * m.inv_dims[2]);
     V3 const hi = v3(float(b1[0]) * m.inv_dims[0], float(b1[1]) * m.inv_dims[1], float(b1[2]) * m.inv_dims[2]);
     float hit_t;
@@ -197,12 +189,8 @@ __device__ inline bool gridtree_intersect(Medium_view const& m, Tray& r, Medium_
         r.max_t = r.min_t;
         return false;
     }
-    uint32_t const node = m.nodes[index];
-    if (Grid_empty == (node >> 1)) {
-        return false;
-    }
-    cm = m.data[node >> 1];
-    return true;
+    cm = leaf;
+    return 0 == (level & Leaf_empty);
 }
 
 // van_de_hulst(g, gs) with gs lerped towards 0 over the range
@@ -297,58 +285,6 @@ __device__ __forceinline__ void coefficients(Medium_view const& m, Channel_cc<NC
     }
 }
 
-// Tracking::tracking (scattering, no emission): true = scattered at t_out.
-// The channel weights are history-aware (the scatter / null probabilities
-// average the channels weighted by the path so far).
-template <int NC, typename Rng>
-__device__ inline bool tracking(Medium_view const& m, Channel_cc<NC> const& cc, Tray const& r,
-                                Medium_cm const& cm, float srs, bool nearest, Rng& rng,
-                                float& t_out, float w[NC]) {
-    float const mt = cm.majorant_mu_a + cm.majorant_mu_s;
-    if (mt < Min_mt) {
-        return false;
-    }
-    float lw[NC];
-    for (int c = 0; c < NC; ++c) {
-        lw[c] = w[c];
-    }
-    float const imt = 1.f / mt;
-    for (float t = r.min_t, d = r.max_t;;) {
-        float const r0 = medium_uniform(rng);
-        t -= logf(1.f - r0) * imt;
-        if (t > d) {
-            for (int c = 0; c < NC; ++c) {
-                w[c] = lw[c];
-            }
-            return false;
-        }
-        float mu_a[NC], mu_s[NC];
-        coefficients<NC>(m, cc, r.point(t), srs, nearest, mu_a, mu_s);
-        float mu_n[NC], msw[NC], mnw[NC];
-        for (int c = 0; c < NC; ++c) {
-            mu_n[c] = mt - (mu_a[c] + mu_s[c]);
-            msw[c]  = mu_s[c] * lw[c];
-            mnw[c]  = mu_n[c] * lw[c];
-        }
-        float const ms = average_channels<NC>(msw);
-        float const mn = average_channels<NC>(mnw);
-        float const ic = 1.f / (ms + mn);
-        float const ps = ms * ic;
-        float const pn = mn * ic;
-        float const r1 = medium_uniform(rng);
-        if ((r1 <= 1.f - pn) & (ps > 0.f)) {
-            for (int c = 0; c < NC; ++c) {
-                w[c] = lw[c] * (mu_s[c] / (mt * ps));
-            }
-            t_out = t;
-            return true;
-        }
-        for (int c = 0; c < NC; ++c) {
-            lw[c] *= mu_n[c] / (mt * pn);
-        }
-    }
-}
-
 template <int NC>
 __device__ __forceinline__ bool all_below(float const w[NC], float e) {
     bool below = true;
@@ -356,51 +292,6 @@ __device__ __forceinline__ bool all_below(float const w[NC], float e) {
         below = below && w[c] < e;
     }
     return below;
-}
-
-// tracking_transmitted with its residual-ratio-tracking branch
-template <int NC, typename Rng>
-__device__ inline bool tracking_transmitted(Medium_view const& m, Channel_cc<NC> const& cc,
-                                            Tray const& r, Medium_cm const& cm, float srs,
-                                            bool nearest, Rng& rng, float w[NC]) {
-    float const mt = cm.majorant_mu_a + cm.majorant_mu_s;
-    if (mt < Min_mt) {
-        return true;
-    }
-    float const minorant = cm.minorant_mu_a + cm.minorant_mu_s;
-    float       control  = 0.f;
-    float       mr       = mt;
-    if (minorant > 0.f) {
-        float const att = expf(-(r.max_t - r.min_t) * minorant);
-        for (int c = 0; c < NC; ++c) {
-            w[c] *= att;
-        }
-        if (all_below<NC>(w, Abort_epsilon)) {
-            return false;
-        }
-        mr = mt - minorant;
-        if (mr < Min_mt) {
-            return true;
-        }
-        control = minorant;
-    }
-    float const imt = 1.f / mr;
-    for (float t = r.min_t, d = r.max_t;;) {
-        float const r0 = medium_uniform(rng);
-        t -= logf(1.f - r0) * imt;
-        if (t > d) {
-            return true;
-        }
-        float mu_a[NC], mu_s[NC];
-        coefficients<NC>(m, cc, r.point(t), srs, nearest, mu_a, mu_s);
-        for (int c = 0; c < NC; ++c) {
-            float const mu_t = (mu_a[c] + mu_s[c]) - control;
-            w[c] *= imt * (mr - mu_t);
-        }
-        if (all_below<NC>(w, Abort_epsilon)) {
-            return false;
-        }
-    }
 }
 
 // Texture-space ray of a world segment [t0, t1] (the part inside the box).
@@ -452,78 +343,189 @@ __device__ inline bool box_overlap(Medium_view const& m, V3 o, V3 d, float min_t
     return t0 < t1;
 }
 
-// Tracking_multi::integrate for one segment (tracking_multi.cpp:101-162):
-// 1 scattered at t_out, 0 passed, 2 aborted (every channel of w below
-// Abort_epsilon, scattered or not).  w multiplies the throughput.
-template <int NC, typename Rng>
-__device__ inline int track_segment(Medium_view const& m, Channel_cc<NC> const& cc, V3 o, V3 d,
-                                    float t0, float t1, uint32_t depth, bool nearest, Rng& rng,
-                                    float& t_out, float w[NC]) {
-    Tray        r     = texture_ray(m, o, d, t0, t1);
-    float const srs   = similarity_scale(m.g, depth);
-    int         event = 0;
-    for (int c = 0; c < NC; ++c) {
-        w[c] = 1.f;
-    }
-    for (float const end = t1; r.min_t < end;) {
-        Medium_cm cm;
-        if (gridtree_intersect(m, r, cm)) {
-            cm.minorant_mu_s *= srs;
-            cm.majorant_mu_s *= srs;
-            if (tracking<NC>(m, cc, r, cm, srs, nearest, rng, t_out, w)) {
-                event = 1;
-                break;
-            }
+// One segment's walk through the medium as steps that a wave's lanes can
+// take in any order: Walk_cell enters the next majorant cell and draws the
+// first distance in it, Walk_collide evaluates a collision and draws the
+// next.
+//   Transmit false  Tracking_multi::integrate (tracking_multi.cpp:101-162)
+//                   with Tracking::tracking (tracking.cpp:328-375:
+//                   scattering, no emission; the channel weights are
+//                   history-aware, the scatter / null probabilities average
+//                   the channels weighted by the path so far)
+//   Transmit true   Tracking::transmittance with tracking_transmitted and
+//                   its residual-ratio-tracking branch (tracking.cpp:32-129)
+enum Walk_state : uint32_t {
+    Walk_cell,
+    Walk_collide,
+    Walk_done,     // left the segment
+    Walk_scatter,  // at t
+    Walk_abort     // Transmit: every channel of w below Abort_epsilon
+};
+
+template <int NC, bool Transmit>
+struct Walk {
+    Tray           r;
+    float          end;
+    float          t;        // the pending collision
+    float          mt;       // the cell's majorant, less the control
+    float          imt;
+    float          control;  // Transmit: the cell's minorant
+    float          srs;
+    float          w[NC];    // multiplies the throughput
+    bool           nearest;
+
+    __device__ __forceinline__ uint32_t start(Medium_view const& m, V3 o, V3 d, float t0, float t1,
+                                              uint32_t depth, bool nearest_) {
+        r       = texture_ray(m, o, d, t0, t1);
+        end     = t1;
+        srs     = similarity_scale(m.g, depth);
+        nearest = nearest_;
+        for (int c = 0; c < NC; ++c) {
+            w[c] = 1.f;
         }
+        return r.min_t < end ? Walk_cell : Walk_done;
+    }
+
+    __device__ __forceinline__ uint32_t leave_cell() {
         r.min_t = offset_f(r.max_t);
         r.max_t = end;
+        return r.min_t < end ? Walk_cell : Walk_done;
     }
-    return all_below<NC>(w, Abort_epsilon) ? 2 : event;
-}
 
+    template <typename Rng>
+    __device__ __forceinline__ uint32_t enter_cell(Medium_view const& m, Rng& rng) {
+        Medium_cm cm;
+        if (!gridtree_intersect(m, r, cm)) {
+            return leave_cell();
+        }
+        cm.minorant_mu_s *= srs;
+        cm.majorant_mu_s *= srs;
+        mt = cm.majorant_mu_a + cm.majorant_mu_s;
+        if (mt < Min_mt) {
+            return leave_cell();
+        }
+        if constexpr (Transmit) {
+            float const minorant = cm.minorant_mu_a + cm.minorant_mu_s;
+            control              = 0.f;
+            if (minorant > 0.f) {
+                float const att = expf(-(r.max_t - r.min_t) * minorant);
+                for (int c = 0; c < NC; ++c) {
+                    w[c] *= att;
+                }
+                if (all_below<NC>(w, Abort_epsilon)) {
+                    return Walk_abort;
+                }
+                mt -= minorant;
+                if (mt < Min_mt) {
+                    return leave_cell();
+                }
+                control = minorant;
+            }
+        }
+        imt = 1.f / mt;
+        t   = r.min_t;
+        return fly(rng);
+    }
+
+    template <typename Rng>
+    __device__ __forceinline__ uint32_t fly(Rng& rng) {
+        float const r0 = medium_uniform(rng);
+        t -= logf(1.f - r0) * imt;
+        return t > r.max_t ? leave_cell() : uint32_t(Walk_collide);
+    }
+
+    template <typename Rng>
+    __device__ __forceinline__ uint32_t collide(Medium_view const& m, Channel_cc<NC> const& cc,
+                                                Rng& rng) {
+        float mu_a[NC], mu_s[NC];
+        coefficients<NC>(m, cc, r.point(t), srs, nearest, mu_a, mu_s);
+        if constexpr (Transmit) {
+            for (int c = 0; c < NC; ++c) {
+                float const mu_t = (mu_a[c] + mu_s[c]) - control;
+                w[c] *= imt * (mt - mu_t);
+            }
+            if (all_below<NC>(w, Abort_epsilon)) {
+                return Walk_abort;
+            }
+        } else {
+            float mu_n[NC], msw[NC], mnw[NC];
+            for (int c = 0; c < NC; ++c) {
+                mu_n[c] = mt - (mu_a[c] + mu_s[c]);
+                msw[c]  = mu_s[c] * w[c];
+                mnw[c]  = mu_n[c] * w[c];
+            }
+            float const ms = average_channels<NC>(msw);
+            float const mn = average_channels<NC>(mnw);
+            float const ic = 1.f / (ms + mn);
+            float const ps = ms * ic;
+            float const pn = mn * ic;
+            float const r1 = medium_uniform(rng);
+            if ((r1 <= 1.f - pn) & (ps > 0.f)) {
+                for (int c = 0; c < NC; ++c) {
+                    w[c] *= mu_s[c] / (mt * ps);
+                }
+                return Walk_scatter;
+            }
+            for (int c = 0; c < NC; ++c) {
+                w[c] *= mu_n[c] / (mt * pn);
+            }
+        }
+        return fly(rng);
+    }
+
+    // the event of a finished Transmit false walk: 1 scattered at t, 0
+    // passed, 2 absorbed (every channel of w below Abort_epsilon)
+    __device__ __forceinline__ int event(uint32_t state) const {
+        return all_below<NC>(w, Abort_epsilon) ? 2 : Walk_scatter == state ? 1 : 0;
+    }
+
+    // all steps of one walk
+    template <typename Rng>
+    __device__ uint32_t run(uint32_t state, Medium_view const& m, Channel_cc<NC> const& cc, Rng& rng) {
+        while (state <= Walk_collide) {
+            state = Walk_cell == state ? enter_cell(m, rng) : collide(m, cc, rng);
+        }
+        return state;
+    }
+};
+
+// track_segment: 1 scattered at t_out, 0 passed, 2 absorbed
 template <typename Rng>
 __device__ inline int track_segment(Medium_view const& m, V3 o, V3 d, float t0, float t1,
                                     uint32_t depth, bool nearest, Rng& rng, float& t_out,
                                     float w[3]) {
-    return track_segment<3>(m, rgb_channels(m), o, d, t0, t1, depth, nearest, rng, t_out, w);
+    Walk<3, false> k;
+    uint32_t const state = k.run(k.start(m, o, d, t0, t1, depth, nearest), m, rgb_channels(m), rng);
+    for (int c = 0; c < 3; ++c) {
+        w[c] = k.w[c];
+    }
+    if (Walk_scatter == state) {
+        t_out = k.t;
+    }
+    return k.event(state);
+}
+
+// Whether anything is tracked on a shadow ray's segment inside the box.
+__device__ __forceinline__ bool transmits_freely(float t0, float t1) {
+    return offset_f(t0) >= t1;
 }
 
 // Tracking::transmittance for the part of a segment inside the box:
 // false = blocked (tr below Abort_epsilon), else tr.
-template <int NC, typename Rng>
-__device__ inline bool transmittance(Medium_view const& m, Channel_cc<NC> const& cc, V3 o, V3 d,
-                                     float t0, float t1, uint32_t depth, bool nearest, Rng& rng,
-                                     float tr[NC]) {
-    for (int c = 0; c < NC; ++c) {
-        tr[c] = 1.f;
-    }
-    if (offset_f(t0) >= t1) {
-        return true;
-    }
-    Tray        r   = texture_ray(m, o, d, t0, t1);
-    float const srs = similarity_scale(m.g, depth);
-    for (float const end = t1; r.min_t < end;) {
-        Medium_cm cm;
-        if (gridtree_intersect(m, r, cm)) {
-            cm.minorant_mu_s *= srs;
-            cm.majorant_mu_s *= srs;
-            if (!tracking_transmitted<NC>(m, cc, r, cm, srs, nearest, rng, tr)) {
-                for (int c = 0; c < NC; ++c) {
-                    tr[c] = 0.f;
-                }
-                return false;
-            }
-        }
-        r.min_t = offset_f(r.max_t);
-        r.max_t = end;
-    }
-    return true;
-}
-
 template <typename Rng>
 __device__ inline bool transmittance(Medium_view const& m, V3 o, V3 d, float t0, float t1,
                                      uint32_t depth, bool nearest, Rng& rng, float tr[3]) {
-    return transmittance<3>(m, rgb_channels(m), o, d, t0, t1, depth, nearest, rng, tr);
+    Walk<3, true> k;
+    uint32_t      state = Walk_done;
+    if (transmits_freely(t0, t1)) {
+        tr[0] = tr[1] = tr[2] = 1.f;
+        return true;
+    }
+    state = k.run(k.start(m, o, d, t0, t1, depth, nearest), m, rgb_channels(m), rng);
+    for (int c = 0; c < 3; ++c) {
+        tr[c] = Walk_abort == state ? 0.f : k.w[c];
+    }
+    return Walk_abort != state;
 }
 
 }  // namespace mi::dev

@@ -48,6 +48,7 @@
 #include "medium.hpp"
 #include "spectral.hpp"
 #include "render.hpp"
+#include "claims.hpp"
 #include "trace.hpp"
 
 #include <hip/hip_runtime.h>
@@ -84,7 +85,9 @@ constexpr uint32_t C_next       = 6 * Counter_line;  // regenerating: the next s
 constexpr uint32_t C_resolve    = 7 * Counter_line;  // the vertices whose shadow rays are resolved
 constexpr uint32_t C_done0      = 8 * Counter_line;  // regenerating: paths that ended this bounce, by queue
 constexpr uint32_t C_claims     = 10 * Counter_line; // the traversals' ray claims
-constexpr uint32_t Num_counters = C_claims + Counter_words;
+constexpr uint32_t C_track      = C_claims + Counter_words;  // medium_track's claims
+constexpr uint32_t C_transmit   = C_track + Counter_words;   // shadow_transmit's
+constexpr uint32_t Num_counters = C_transmit + Counter_words;
 
 // No kernel of a bounce exists to clear or add up counters (four of one
 // thread each, 4.7 us apiece, were 0.17 ms of a 1.9 ms frame of nine
@@ -92,7 +95,8 @@ constexpr uint32_t Num_counters = C_claims + Counter_words;
 // of a kernel that runs when the last reader is done and the next writer has
 // not begun:
 //   claims          shade (after the closest hits), shadow_resolve (after the
-//                   shadow rays), for the traversal that follows
+//                   shadow rays), for the traversal that follows; the
+//                   medium kernels' own by shade
 //   queue in_q      nee, which adds it to the totals and leaves its length in
 //                   C_resolve; the next bounce fills it
 //   shadow queue    shadow_resolve; nee adds it to the totals
@@ -265,6 +269,7 @@ struct Wave {
     Nee_vertex* nee;         // per queue entry whose vertex picked lights
     Pick_slot*  picks;       // per shadow entry: the light it goes to
     uint32_t* counters;
+    uint32_t  spread_waves;  // waves a small queue of walks fills first (Claims)
     // guiding
     float        fraction;      // probability of sampling the guide
     float const* guide_raw;     // 32 network outputs per queue entry
@@ -687,9 +692,9 @@ __device__ mi_ray start_path(Wave const& w, uint32_t k, uint32_t slot) {
 }
 
 // The traversal that follows hands out its rays from the start.
-__device__ __forceinline__ void clear_claims(Wave const& w) {
+__device__ __forceinline__ void clear_claims(Wave const& w, uint32_t at = C_claims) {
     if (0 == blockIdx.x && threadIdx.x < Claim_parts) {
-        w.counters[C_claims + threadIdx.x * Claim_stride] = 0;
+        w.counters[at + threadIdx.x * Claim_stride] = 0;
     }
 }
 
@@ -703,6 +708,7 @@ __global__ void __launch_bounds__(256) raygen(Wave w) {
         w.ray_path[0][p] = p;
     }
     clear_claims(w);
+    clear_claims(w, C_track);
     if (0 == p) {
         w.counters[C_queue0]                = live;
         w.counters[C_queue0 + Counter_line] = 0;
@@ -724,54 +730,135 @@ __device__ __forceinline__ dev::Channel_cc<4> wavelength_channels(dev::Medium_vi
     return cc;
 }
 
+// The walks of a wave through the medium, shared by medium_track and
+// shadow_transmit.  A walk is a few to a hundred cells and collisions; one
+// walk a lane, cells and collisions in nested loops, kept 13 to 15 of 64
+// lanes busy.  Here a wave steps the lanes of one kind at a time, the kind
+// more of them wait for, and once Service_lanes have ended their walks they
+// deliver the results and take new items.  Bound by VALU issue at the first
+// depths (16 to 20 lanes: a bounce has no more walks than the chip has lanes,
+// so few waves find new items) and by the chain of the longest walk at the
+// later ones.
+// A frame of a 256^3 cloud, 512x512x4 paths: 3.81 ms with nested loops.
+// Workgroups a CU and rays a claim: 8 and 64 took 3.32 ms a frame, 4 and 64
+// 3.20 ms, 4 and 16 3.12 ms, 2 and 16 3.41 ms; 8 to 48 service lanes are
+// within 1 %.
+constexpr uint32_t Service_lanes = 16;
+constexpr uint32_t Walk_blocks   = 4;   // workgroups a CU
+constexpr uint32_t Walk_batch    = 16;  // items a claim
+constexpr uint32_t Walk_idle     = 8;   // beside dev::Walk_state: no walk
+
+// take(i): the lane takes item i; serve(): ends a lane's finished walk and
+// readies its next one (its item's, or Walk_idle).  State of the walks in
+// walk, cc, rng, state of every lane.
+template <int NC, bool Transmit, class Take, class Serve>
+__device__ __forceinline__ void walk_items(Wave const& w, uint32_t count, uint32_t* claim_counters,
+                                           dev::Walk<NC, Transmit>& walk,
+                                           dev::Channel_cc<NC>& cc, Rng& rng, uint32_t& state,
+                                           bool& taken, Take take, Serve serve) {
+    uint32_t const lane  = threadIdx.x & 63;
+    uint32_t const waves = (gridDim.x * blockDim.x) >> 6;
+    uint32_t const wave  = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    Claims         claims;
+    uint32_t       pool = 0, pool_end = 0;
+    claims.init(wave, waves, w.spread_waves, count, pool, pool_end);
+    bool more = true;  // wave-uniform
+    for (;;) {
+        uint64_t const busy = __ballot(state <= dev::Walk_collide);
+        if (0 == busy || (more && 64 - __popcll(busy) >= int(Service_lanes))) {
+            if (state > dev::Walk_collide && taken) {
+                serve();
+            }
+            uint64_t const free = __ballot(!taken);
+            if (more && free) {
+                if (pool == pool_end) {
+                    more = claims.next(claim_counters, count, Walk_batch, lane, pool, pool_end);
+                }
+                uint32_t const rank = uint32_t(__popcll(free & ((uint64_t(1) << lane) - 1)));
+                uint32_t const left = more ? pool_end - pool : 0u;
+                if (!taken && rank < left) {
+                    taken = true;
+                    take(pool + rank);
+                    serve();
+                }
+                pool += min(uint32_t(__popcll(free)), left);
+            }
+            if (!more && 0 == __ballot(taken)) {
+                break;
+            }
+            continue;
+        }
+        uint64_t const cells = __ballot(dev::Walk_cell == state);
+        if (2 * __popcll(cells) >= __popcll(busy)) {
+            if (dev::Walk_cell == state) {
+                state = walk.enter_cell(w.medium, rng);
+            }
+        } else if (dev::Walk_collide == state) {
+            state = walk.collide(w.medium, cc, rng);
+        }
+    }
+}
+
 // Tracking_multi::integrate for every queued ray: the part of the ray before
 // its surface hit that lies in the medium box is tracked; the tracking weight
 // multiplies the path throughput, and a scattering point replaces the hit.
 // Spectral: the channels are the path's four wavelengths.
 template <bool Spectral>
 __device__ __forceinline__ void medium_track_queue(Wave const& w, uint32_t in_q) {
-    constexpr int  NC     = Spectral ? 4 : 3;
-    uint32_t const count  = w.counters[C_queue0 + Counter_line * in_q];
-    uint32_t const stride = gridDim.x * blockDim.x;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride) {
-        mi_ray const r     = w.rays[in_q][i];
-        Hit const    h     = load_hit(w, i);
-        V3 const     o     = v3(r.origin[0], r.origin[1], r.origin[2]);
-        V3 const     d     = v3(r.direction[0], r.direction[1], r.direction[2]);
-        uint32_t     event = Medium_none;
-        float        t0, t1;
-        if (dev::box_overlap(w.medium, o, d, r.min_t, h.t, t0, t1)) {
-            uint32_t const p     = w.ray_path[in_q][i];
-            Path           path  = w.paths[p];
-            float          t_out = 0.f;
-            float          tw[NC];
-            int            e;
-            if constexpr (Spectral) {
-                float2 sp = w.path_spec[p];
-                e = dev::track_segment<4>(w.medium, wavelength_channels(w.medium, sp.y), o, d, t0,
-                                          t1, path.depth, 0 != (path.flags & Flag_nearest),
-                                          path.rng, t_out, tw);
-                sp.x *= tw[3];
-                w.path_spec[p] = sp;
+    constexpr int       NC    = Spectral ? 4 : 3;
+    uint32_t const      count = w.counters[C_queue0 + Counter_line * in_q];
+    dev::Walk<NC, false> walk;
+    dev::Channel_cc<NC> cc = {};
+    Rng                 rng;
+    uint32_t            state = Walk_idle;
+    uint32_t            item  = 0;
+    bool                taken = false;
+    auto const take = [&](uint32_t i) { item = i; };
+    auto const serve = [&] {
+        uint32_t const i = item;
+        mi_ray const   r = w.rays[in_q][i];
+        V3 const       o = v3(r.origin[0], r.origin[1], r.origin[2]);
+        V3 const       d = v3(r.direction[0], r.direction[1], r.direction[2]);
+        uint32_t const p = w.ray_path[in_q][i];
+        Path&          path = w.paths[p];
+        if (Walk_idle == state) {
+            float t0, t1;
+            if (dev::box_overlap(w.medium, o, d, r.min_t, load_hit(w, i).t, t0, t1)) {
+                rng   = path.rng;
+                state = walk.start(w.medium, o, d, t0, t1, path.depth, 0 != (path.flags & Flag_nearest));
+                if constexpr (Spectral) {
+                    cc = wavelength_channels(w.medium, w.path_spec[p].y);
+                } else {
+                    cc = dev::rgb_channels(w.medium);
+                }
             } else {
-                e = dev::track_segment(w.medium, o, d, t0, t1, path.depth,
-                                       0 != (path.flags & Flag_nearest), path.rng, t_out, tw);
+                w.medium_event[i] = Medium_none;
+                taken             = false;
             }
-            for (int c = 0; c < 3; ++c) {
-                path.throughput[c] *= tw[c];
-            }
-            if (1 == e) {
-                event                  = Medium_scatter;
-                w.medium_p[3 * i + 0] = o.x + t_out * d.x;
-                w.medium_p[3 * i + 1] = o.y + t_out * d.y;
-                w.medium_p[3 * i + 2] = o.z + t_out * d.z;
-            } else if (2 == e) {
-                event = Medium_absorbed;
-            }
-            w.paths[p] = path;
+            return;
+        }
+        int const e     = walk.event(state);
+        uint32_t  event = Medium_none;
+        for (int c = 0; c < 3; ++c) {
+            path.throughput[c] *= walk.w[c];
+        }
+        if constexpr (Spectral) {
+            w.path_spec[p].x *= walk.w[3];
+        }
+        path.rng = rng;
+        if (1 == e) {
+            event                  = Medium_scatter;
+            w.medium_p[3 * i + 0] = o.x + walk.t * d.x;
+            w.medium_p[3 * i + 1] = o.y + walk.t * d.y;
+            w.medium_p[3 * i + 2] = o.z + walk.t * d.z;
+        } else if (2 == e) {
+            event = Medium_absorbed;
         }
         w.medium_event[i] = event;
-    }
+        state             = Walk_idle;
+        taken             = false;
+    };
+    walk_items(w, count, w.counters + C_track, walk, cc, rng, state, taken, take, serve);
 }
 
 __global__ void __launch_bounds__(256) medium_track(Wave w, uint32_t in_q) {
@@ -840,6 +927,10 @@ __device__ __forceinline__ void shade_queue(Wave const& w, uint32_t in_q) {
     uint32_t const out_q  = in_q ^ 1;
     uint32_t const stride = gridDim.x * blockDim.x;
     clear_claims(w);
+    if (w.medium.present) {
+        clear_claims(w, C_track);
+        clear_claims(w, C_transmit);
+    }
 
     // block-uniform trip count: every lane reaches the wave-wide queue appends
     for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
@@ -1480,14 +1571,7 @@ __global__ void __launch_bounds__(256) nee_spectral(Wave w, uint32_t in_q) {
 
 // Adds the unoccluded light contributions of every vertex shaded this
 // bounce to its path, in the order the lights were picked.
-// With a medium, the part of each unoccluded shadow ray inside its box is
-// attenuated by ratio tracking (Worker::transmitted: visibility, then
-// transmittance, rendering_worker.cpp:143-153), drawing from the path's
-// generator after the vertex's direction sample.
-// Spectral: transmittance per wavelength, then the film's response.
-template <bool Spectral>
-__device__ __forceinline__ void shadow_resolve_queue(Wave const& w, uint32_t in_q) {
-    constexpr int  NC     = Spectral ? 4 : 3;
+__global__ void __launch_bounds__(256) shadow_resolve(Wave w, uint32_t in_q) {
     uint32_t const count  = w.counters[C_resolve];
     uint32_t const stride = gridDim.x * blockDim.x;
     clear_claims(w);
@@ -1499,67 +1583,139 @@ __device__ __forceinline__ void shadow_resolve_queue(Wave const& w, uint32_t in_
         if (0 == range.y) {
             continue;
         }
-        uint32_t const path        = w.ray_path[in_q][i];
-        Path* const    p           = &w.paths[path];
-        Rng            rng         = p->rng;
-        float          radiance[3] = {p->radiance[0], p->radiance[1], p->radiance[2]};
+        Path* const p           = &w.paths[w.ray_path[in_q][i]];
+        float       radiance[3] = {p->radiance[0], p->radiance[1], p->radiance[2]};
         spectral::Wavelengths wl;
-        dev::Channel_cc<NC>   cc;
-        if constexpr (Spectral) {
-            wl.set(w.path_spec[path].y);
-            wl.upsample4(w.medium.cc_a, cc.a);
-            wl.upsample4(w.medium.cc_s, cc.s);
-        } else {
-            cc = dev::rgb_channels(w.medium);
+        if (w.spectral) {
+            wl.set(w.path_spec[w.ray_path[in_q][i]].y);
         }
         for (uint32_t k = 0; k < range.y; ++k) {
             if (w.occluded[range.x + k]) {
                 continue;
             }
-            Shadow const s = w.shadows[range.x + k];
-            float        tr[NC];
-            for (int c = 0; c < NC; ++c) {
-                tr[c] = 1.f;
-            }
-            if (w.medium.present) {
-                mi_ray const r = w.shadow_rays[range.x + k];
-                V3 const     o = v3(r.origin[0], r.origin[1], r.origin[2]);
-                V3 const     d = v3(r.direction[0], r.direction[1], r.direction[2]);
-                float        t0, t1;
-                if (r.min_t < r.max_t && dev::box_overlap(w.medium, o, d, r.min_t, r.max_t, t0, t1)) {
-                    if (!dev::transmittance<NC>(w.medium, cc, o, d, t0, t1, w.nee[i].depth,
-                                                0 != (p->flags & Flag_nearest), rng, tr)) {
-                        continue;
-                    }
-                }
-            }
-            if constexpr (Spectral) {
-                float const c4[4] = {tr[0] * s.contrib[0], tr[1] * s.contrib[1],
-                                     tr[2] * s.contrib[2], tr[3] * w.shadow_c4[range.x + k]};
-                float       rgb[3];
+            Shadow const s      = w.shadows[range.x + k];
+            float        rgb[3] = {s.contrib[0], s.contrib[1], s.contrib[2]};
+            if (w.spectral) {
+                float const c4[4] = {s.contrib[0], s.contrib[1], s.contrib[2], w.shadow_c4[range.x + k]};
                 wl.to_rgb(w.spec_minv, c4, rgb);
-                for (int c = 0; c < 3; ++c) {
-                    radiance[c] += rgb[c];
-                }
-            } else {
-                for (int c = 0; c < 3; ++c) {
-                    radiance[c] += tr[c] * s.contrib[c];
-                }
+            }
+            for (int c = 0; c < 3; ++c) {
+                radiance[c] += rgb[c];
             }
         }
         for (int c = 0; c < 3; ++c) {
             p->radiance[c] = radiance[c];
         }
-        p->rng = rng;
     }
 }
 
-__global__ void __launch_bounds__(256) shadow_resolve(Wave w, uint32_t in_q) {
-    shadow_resolve_queue<false>(w, in_q);
+// shadow_resolve with a medium: the part of each unoccluded shadow ray inside
+// its box is attenuated by ratio tracking (Worker::transmitted: visibility,
+// then transmittance, rendering_worker.cpp:143-153), drawing from the path's
+// generator after the vertex's direction sample.
+// Spectral: transmittance per wavelength, then the film's response.
+template <bool Spectral>
+__device__ __forceinline__ void shadow_transmit_queue(Wave const& w, uint32_t in_q) {
+    constexpr int  NC    = Spectral ? 4 : 3;
+    uint32_t const count = w.counters[C_resolve];
+    clear_claims(w);
+    if (0 == blockIdx.x && 0 == threadIdx.x) {
+        w.counters[C_shadow] = 0;
+    }
+    dev::Walk<NC, true> walk;
+    dev::Channel_cc<NC> cc = {};
+    Rng                 rng;
+    uint32_t            state = Walk_idle;
+    uint32_t            item  = 0;
+    uint32_t            at = 0, last = 0;  // the vertex's shadow rays left
+    bool                taken = false;
+    float               radiance[3] = {0.f, 0.f, 0.f};
+
+    auto const add = [&](uint32_t path, float const tr[NC]) {
+        Shadow const s = w.shadows[at];
+        if constexpr (Spectral) {
+            float const c4[4] = {tr[0] * s.contrib[0], tr[1] * s.contrib[1], tr[2] * s.contrib[2],
+                                 tr[3] * w.shadow_c4[at]};
+            spectral::Wavelengths wl;
+            wl.set(w.path_spec[path].y);
+            float rgb[3];
+            wl.to_rgb(w.spec_minv, c4, rgb);
+            for (int c = 0; c < 3; ++c) {
+                radiance[c] += rgb[c];
+            }
+        } else {
+            for (int c = 0; c < 3; ++c) {
+                radiance[c] += tr[c] * s.contrib[c];
+            }
+        }
+    };
+    auto const take = [&](uint32_t i) {
+        uint2 const range = w.shadow_range[i];
+        if (0 == range.y) {
+            taken = false;
+            return;
+        }
+        item = i;
+        at   = range.x;
+        last = range.x + range.y;
+        uint32_t const path = w.ray_path[in_q][i];
+        rng                 = w.paths[path].rng;
+        for (int c = 0; c < 3; ++c) {
+            radiance[c] = w.paths[path].radiance[c];
+        }
+        if constexpr (Spectral) {
+            cc = wavelength_channels(w.medium, w.path_spec[path].y);
+        } else {
+            cc = dev::rgb_channels(w.medium);
+        }
+    };
+    auto const serve = [&] {
+        if (!taken) {
+            return;
+        }
+        uint32_t const path = w.ray_path[in_q][item];
+        if (Walk_idle != state) {
+            if (dev::Walk_abort != state) {
+                add(path, walk.w);
+            }
+            ++at;
+            state = Walk_idle;
+        }
+        for (; at < last; ++at) {
+            if (w.occluded[at]) {
+                continue;
+            }
+            mi_ray const r = w.shadow_rays[at];
+            V3 const     o = v3(r.origin[0], r.origin[1], r.origin[2]);
+            V3 const     d = v3(r.direction[0], r.direction[1], r.direction[2]);
+            float        t0, t1;
+            if (r.min_t < r.max_t && dev::box_overlap(w.medium, o, d, r.min_t, r.max_t, t0, t1) &&
+                !dev::transmits_freely(t0, t1)) {
+                state = walk.start(w.medium, o, d, t0, t1, w.nee[item].depth,
+                                   0 != (w.paths[path].flags & Flag_nearest));
+                return;
+            }
+            float one[NC];
+            for (int c = 0; c < NC; ++c) {
+                one[c] = 1.f;
+            }
+            add(path, one);
+        }
+        for (int c = 0; c < 3; ++c) {
+            w.paths[path].radiance[c] = radiance[c];
+        }
+        w.paths[path].rng = rng;
+        taken             = false;
+    };
+    walk_items(w, count, w.counters + C_transmit, walk, cc, rng, state, taken, take, serve);
 }
 
-__global__ void __launch_bounds__(256) shadow_resolve_spectral(Wave w, uint32_t in_q) {
-    shadow_resolve_queue<true>(w, in_q);
+__global__ void __launch_bounds__(256) shadow_transmit(Wave w, uint32_t in_q) {
+    shadow_transmit_queue<false>(w, in_q);
+}
+
+__global__ void __launch_bounds__(256) shadow_transmit_spectral(Wave w, uint32_t in_q) {
+    shadow_transmit_queue<true>(w, in_q);
 }
 
 // Marks every record slot of the wave empty; the shading kernels fill the
@@ -2137,11 +2293,11 @@ void RenderScene::release() {
 
 void RenderScene::release_medium() {
     (void)hipFree(medium_density);
-    (void)hipFree(medium_nodes);
-    (void)hipFree(medium_data);
+    (void)hipFree(medium_levels);
+    (void)hipFree(medium_leaves);
     medium_density = nullptr;
-    medium_nodes   = nullptr;
-    medium_data    = nullptr;
+    medium_levels  = nullptr;
+    medium_leaves  = nullptr;
     medium         = dev::Medium_view{};
 }
 
@@ -2275,16 +2431,39 @@ int32_t set_medium(RenderScene& scene, float const* density, uint32_t const dims
     HostGridtree  tree;
     build_gridtree(density, idims, cc_a, cc_s, tree, MI_MAJORANTS_FLAT == majorants);
 
-    hipError_t e = hipMalloc(&scene.medium_density, n * sizeof(float));
-    if (!e) e = hipMalloc(&scene.medium_nodes, tree.nodes.size() * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&scene.medium_data, std::max<size_t>(tree.data.size(), 1) * sizeof(Medium_cm));
-    if (!e) e = hipMemcpy(scene.medium_density, density, n * sizeof(float), hipMemcpyHostToDevice);
-    if (!e) e = hipMemcpy(scene.medium_nodes, tree.nodes.data(), tree.nodes.size() * sizeof(uint32_t),
-                          hipMemcpyHostToDevice);
-    if (!e && !tree.data.empty()) {
-        e = hipMemcpy(scene.medium_data, tree.data.data(), tree.data.size() * sizeof(Medium_cm),
-                      hipMemcpyHostToDevice);
+    // the leaves per block of the smallest leaf size
+    uint32_t const         split = dev::Log2_cell_dim - dev::Log2_block_dim;
+    uint32_t const         nb[3] = {uint32_t(tree.num_cells[0]) << split, uint32_t(tree.num_cells[1]) << split,
+                                    uint32_t(tree.num_cells[2]) << split};
+    std::vector<uint8_t>   levels(size_t(nb[0]) * nb[1] * nb[2]);
+    std::vector<Medium_cm> leaves(levels.size());
+    for (uint32_t z = 0, i = 0; z < nb[2]; ++z) {
+        for (uint32_t y = 0; y < nb[1]; ++y) {
+            for (uint32_t x = 0; x < nb[0]; ++x, ++i) {
+                uint32_t node  = ((z >> split) * uint32_t(tree.num_cells[1]) + (y >> split)) *
+                                    uint32_t(tree.num_cells[0]) + (x >> split);
+                uint32_t level = 0;
+                while (tree.nodes[node] & 1u) {
+                    ++level;
+                    uint32_t const bit = split - level;
+                    node = (tree.nodes[node] >> 1) + (((x >> bit) & 1u) | (((y >> bit) & 1u) << 1) |
+                                                      (((z >> bit) & 1u) << 2));
+                }
+                uint32_t const data = tree.nodes[node] >> 1;
+                bool const     none = dev::Grid_empty == data;
+                levels[i]           = uint8_t(level | (none ? dev::Leaf_empty : 0u));
+                leaves[i]           = none ? Medium_cm{0.f, 0.f, 0.f, 0.f} : tree.data[data];
+            }
+        }
     }
+
+    hipError_t e = hipMalloc(&scene.medium_density, n * sizeof(float));
+    if (!e) e = hipMalloc(&scene.medium_levels, levels.size());
+    if (!e) e = hipMalloc(&scene.medium_leaves, leaves.size() * sizeof(Medium_cm));
+    if (!e) e = hipMemcpy(scene.medium_density, density, n * sizeof(float), hipMemcpyHostToDevice);
+    if (!e) e = hipMemcpy(scene.medium_levels, levels.data(), levels.size(), hipMemcpyHostToDevice);
+    if (!e) e = hipMemcpy(scene.medium_leaves, leaves.data(), leaves.size() * sizeof(Medium_cm),
+                          hipMemcpyHostToDevice);
     if (e) {
         scene.release_medium();
         return fail(MI_ERR_HIP, "medium upload: %s", hipGetErrorString(e));
@@ -2300,8 +2479,8 @@ int32_t set_medium(RenderScene& scene, float const* density, uint32_t const dims
         m.cc_a[k]      = cc_a[k];
         m.cc_s[k]      = cc_s[k];
     }
-    m.nodes   = scene.medium_nodes;
-    m.data    = scene.medium_data;
+    m.levels  = scene.medium_levels;
+    m.leaves  = scene.medium_leaves;
     m.g       = g;
     m.present = 1;
     return MI_OK;
@@ -3605,6 +3784,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
     w.picks        = static_cast<Pick_slot*>(state.picks);
     w.guide_mix    = state.guide_mix;
     w.counters    = state.counters;
+    w.spread_waves = trace.num_cus;
     w.fraction        = guided ? gs->fraction : 0.f;
     w.guide_raw       = state.guide_raw;
     w.guide_x         = state.guide_x;
@@ -3636,7 +3816,12 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
     uint32_t const    waves     = set.samples_per_pixel / spw;
     uint32_t const    grid_path = std::min<uint32_t>(blocks(num_paths, 256), trace.num_cus * 8);
     uint32_t const    grid_shadow = std::min<uint32_t>(blocks(num_shadow, 256), trace.num_cus * 8);
+    // the medium walks hand out items to resident waves
+    uint32_t const    grid_walk = std::min<uint32_t>(blocks(num_paths, 256), trace.num_cus * Walk_blocks);
     auto const        start     = std::chrono::steady_clock::now();
+
+    void (*const resolve_shadows)(Wave, uint32_t) =
+        !scene.medium.present ? shadow_resolve : spectral ? shadow_transmit_spectral : shadow_transmit;
 
     // traversals with their ray counts on the device: the scene's tree, or
     // the top-level tree over instances
@@ -3674,7 +3859,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             }
             if (scene.medium.present) {
                 hipLaunchKernelGGL(spectral ? medium_track_spectral : medium_track,
-                                   dim3(grid_path), dim3(256), 0, s, w, q);
+                                   dim3(grid_walk), dim3(256), 0, s, w, q);
             }
             if (guided && d < guide_depth) {
                 hipLaunchKernelGGL(guide_inputs, dim3(grid_path), dim3(256), 0, s, w, q);
@@ -3698,8 +3883,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             if (int32_t const st = trace_any(); st) {
                 return st;
             }
-            hipLaunchKernelGGL(spectral ? shadow_resolve_spectral : shadow_resolve,
-                               dim3(grid_path), dim3(256), 0, s, w, q);
+            hipLaunchKernelGGL(resolve_shadows, dim3(scene.medium.present ? grid_walk : grid_path), dim3(256), 0, s, w, q);
             q ^= 1;
         }
         if (sensor) {
@@ -3739,7 +3923,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             return st;
         }
         if (scene.medium.present) {
-            hipLaunchKernelGGL(spectral ? medium_track_spectral : medium_track, dim3(grid_path),
+            hipLaunchKernelGGL(spectral ? medium_track_spectral : medium_track, dim3(grid_walk),
                                dim3(256), 0, s, w, q);
         }
         hipLaunchKernelGGL(spectral ? shade_spectral : shade, dim3(grid_path), dim3(256), 0, s, w, q);
@@ -3747,7 +3931,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
         if (int32_t const st = trace_any(); st) {
             return st;
         }
-        hipLaunchKernelGGL(spectral ? shadow_resolve_spectral : shadow_resolve, dim3(grid_path),
+        hipLaunchKernelGGL(resolve_shadows, dim3(scene.medium.present ? grid_walk : grid_path),
                            dim3(256), 0, s, w, q);
         hipLaunchKernelGGL(regenerate, dim3(grid_path), dim3(256), 0, s, w, q ^ 1);
         return MI_OK;

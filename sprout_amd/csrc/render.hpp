@@ -104,8 +104,8 @@ struct RenderScene {
     Emitter_work                 emitter_work;
     // participating medium in an axis-aligned box (none while density is null)
     float*           medium_density = nullptr;  // nx * ny * nz, x fastest
-    uint32_t*        medium_nodes   = nullptr;  // majorant gridtree
-    Medium_cm*       medium_data    = nullptr;
+    uint8_t*         medium_levels  = nullptr;  // the majorant gridtree's leaves, per block
+    Medium_cm*       medium_leaves  = nullptr;
     dev::Medium_view medium{};
     // instanced scenes: the mesh instances and, last, the triangles above
     // (emitters and other world-space triangles) as one more instance
