@@ -14,11 +14,12 @@
 //           pass through LDS, the output layer stores to memory; weights
 //           are loaded once per workgroup and the grid strides over tiles.
 // gradient  a workgroup of 4 waves takes 64 samples at a time: each wave runs
-//           forward and backward for its 16 (activations and pre-activation
-//           gradients kept in LDS), then the 4 waves split the 96 16x16 tiles
-//           of the weight gradients (depth = the 64 samples) and keep them in
-//           registers across all chunks; partial sums per workgroup are
-//           reduced in a fixed order, so gradients are deterministic.
+//           forward and backward for its 16, whose activations and
+//           pre-activation gradients also go to LDS transposed; then the 4
+//           waves split the 96 16x16 tiles of the weight gradients (depth =
+//           the 64 samples) and keep them in registers across all chunks;
+//           partial sums per workgroup are reduced in a fixed order, so
+//           gradients are deterministic.
 // adam      one thread per parameter; refreshes the bf16 W^T copy.
 
 #include "common.hpp"
@@ -37,7 +38,6 @@ namespace {
 
 using namespace guide;
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // LDS row strides (elements), padded against bank conflicts; multiples of 4
@@ -69,12 +69,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ bf16x4 load4(uint16_t const* p) {
-    return *reinterpret_cast<bf16x4 const*>(p);
-}
-
-
-
 // gfx950's double-depth product: 16 x 16 x 32, each lane supplying eight
 // consecutive depth elements.  Lane (r, q) gives A[r][8q + t] and
 // B[8q + t][r], t = 0..7; whatever order the unit adds the 32 depth terms
@@ -100,24 +94,30 @@ __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 
 struct Weights {
-    uint16_t w1[Hidden * S_feat];
-    uint16_t w2[Hidden * S_hid];
-    uint16_t w3[Hidden * S_hid];
-    uint16_t w4[Num_out * S_hid];
+    alignas(16) uint16_t w1[Hidden * S_feat];
+    alignas(16) uint16_t w2[Hidden * S_hid];
+    alignas(16) uint16_t w3[Hidden * S_hid];
+    alignas(16) uint16_t w4[Num_out * S_hid];
     float    b[3 * Hidden + Num_out];
 };
 
+// Rows of `cols` weights to LDS rows of `stride`, 16 bytes a load (2-byte
+// loads took 11 us of a workgroup's start).
+template <int Rows, int Cols, int Stride>
+__device__ __forceinline__ void load_rows(uint16_t* dst, uint16_t const* src) {
+    static_assert(Cols % 8 == 0 && Stride % 8 == 0, "16-byte pieces");
+    for (int i = threadIdx.x; i < Rows * (Cols / 8); i += blockDim.x) {
+        *reinterpret_cast<uint4*>(dst + (i / (Cols / 8)) * Stride + 8 * (i % (Cols / 8))) =
+            reinterpret_cast<uint4 const*>(src)[i];
+    }
+}
+
 __device__ void load_weights(Weights& s, uint16_t const* wt, float const* params) {
-    for (int i = threadIdx.x; i < Hidden * Feat_pad; i += blockDim.x) {
-        s.w1[(i / Feat_pad) * S_feat + i % Feat_pad] = wt[T_w1 + i];
-    }
-    for (int i = threadIdx.x; i < Hidden * Hidden; i += blockDim.x) {
-        s.w2[(i / Hidden) * S_hid + i % Hidden] = wt[T_w2 + i];
-        s.w3[(i / Hidden) * S_hid + i % Hidden] = wt[T_w3 + i];
-    }
-    for (int i = threadIdx.x; i < Num_out * Hidden; i += blockDim.x) {
-        s.w4[(i / Hidden) * S_hid + i % Hidden] = wt[T_w4 + i];
-    }
+    static_assert(T_w1 % 8 == 0 && T_w2 % 8 == 0 && T_w3 % 8 == 0 && T_w4 % 8 == 0, "16-byte pieces");
+    load_rows<Hidden, Feat_pad, S_feat>(s.w1, wt + T_w1);
+    load_rows<Hidden, Hidden, S_hid>(s.w2, wt + T_w2);
+    load_rows<Hidden, Hidden, S_hid>(s.w3, wt + T_w3);
+    load_rows<Num_out, Hidden, S_hid>(s.w4, wt + T_w4);
     for (int i = threadIdx.x; i < Hidden; i += blockDim.x) {
         s.b[i]              = params[Off_b1 + i];
         s.b[Hidden + i]     = params[Off_b2 + i];
@@ -128,40 +128,11 @@ __device__ void load_weights(Weights& s, uint16_t const* wt, float const* params
     }
 }
 
-// Features of 16 queries into X [16][S_feat]; row m = query row0 + m, rows
-// past n are zero.  x: 9 inputs per query in [0,1]; feature (i, j) is
-// sin / cos of pi (freq[i][j] x_i), the product rounded to fp32.
-__device__ void features(float const* x, float const* freq, uint32_t row0, uint32_t n, uint16_t* X) {
-    int const      lane = threadIdx.x & 63;
-    int const      m    = lane & 15;
-    int const      g    = lane >> 4;
-    uint32_t const row  = row0 + m;
-    for (int i = g; i < Num_in; i += 4) {
-        float const v = row < n ? x[size_t(row) * Num_in + i] : 0.f;
-        for (int j = 0; j < Num_freq; ++j) {
-            // sin(pi f) = sin(2 pi (f / 2)): the hardware sine of the
-            // fraction of f / 2 turns (f / 2 and its fraction are exact)
-            float const f   = freq[i * Num_freq + j] * v;
-            float const h   = 0.5f * f;
-            float const rev = h - floorf(h);
-            float const s   = row < n ? __builtin_amdgcn_sinf(rev) : 0.f;
-            float const c   = row < n ? __builtin_amdgcn_cosf(rev) : 0.f;
-            // the pair (sin, cos) as one 4-byte store (row and pair offsets are even)
-            *reinterpret_cast<uint32_t*>(X + m * S_feat + 24 * i + 2 * j) = pack_bf16(s, c);
-        }
-    }
-    if (3 == g) {
-        for (int k = Num_feat; k < Feat_pad; ++k) {
-            X[m * S_feat + k] = 0;
-        }
-    }
-}
-
 // Epilogue of a layer: acc[nt][t] is output 16 nt + 4q + t of row r; adds
 // the bias and writes, per Mode, ReLU'd bf16 to H (one 8-byte store per
-// tile), fp32 to F (Mode_f32), or fp32 rows r < rows to global F (Mode_out;
-// float4 stores where F is 16-byte aligned, sf a multiple of 4).
-enum { Mode_relu = 0, Mode_f32 = 1, Mode_out = 2 };
+// tile), or fp32 rows r < rows to global F (Mode_out; float4 stores where F
+// is 16-byte aligned, sf a multiple of 4).
+enum { Mode_relu = 0, Mode_out = 1 };
 
 template <int N, int Mode>
 __device__ __forceinline__ void store_layer(f32x4 const (&acc)[N / 16], float const* bias, int r,
@@ -180,11 +151,6 @@ __device__ __forceinline__ void store_layer(f32x4 const (&acc)[N / 16], float co
             pk.x = pack_bf16(fmaxf(v[0], 0.f), fmaxf(v[1], 0.f));
             pk.y = pack_bf16(fmaxf(v[2], 0.f), fmaxf(v[3], 0.f));
             *reinterpret_cast<uint2*>(H + r * sh + j0) = pk;
-        } else if (Mode_f32 == Mode) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                F[r * sf + j0 + t] = v[t];
-            }
         } else if (r < rows) {
             float* const o = F + size_t(r) * sf + j0;
             if (0 == (reinterpret_cast<uintptr_t>(o) & 15u)) {
@@ -233,7 +199,7 @@ __device__ void layer(uint16_t const* A, int sa, uint16_t const* Wt, int sw, flo
 // B operand of lane (r, q) at depth step ks is features k0 .. k0 + 7, k0 =
 // 32 ks + 8q, of query row0 + r, i.e. (sin, cos) of pi f x_i for i = k0 / 24
 // and the multipliers j0 .. j0 + 3 with j0 = (k0 % 24) / 2 (zero past the
-// 216 features): the values features() writes.  half_freq holds
+// 216 features): the values gradient_kernel forms.  half_freq holds
 // f / 2, and (f / 2) x equals (f x) / 2 for every normal product.  Rows past
 // n run on zero inputs; rows do not mix and theirs are never stored.
 __device__ void layer1_direct(float const* x, float const* half_freq, uint32_t row0, uint32_t n,
@@ -328,18 +294,29 @@ constexpr int Grad_tiles = (Feat_pad / 16) * (Hidden / 16) + 2 * (Hidden / 16) *
                            (Hidden / 16) * (Num_out / 16);  // 56 + 32 + 8 = 96
 constexpr int Tiles_per_wave = Grad_tiles / Grad_waves;      // 24
 
+// Sample-major rows of the transposed operands: the 64 samples of a chunk and
+// padding that puts 16 rows on distinct banks (16-byte reads of 16 lanes).
+constexpr int S_smp = Chunk + 8;  // 72
+constexpr int S_y   = 36;         // fp32 outputs of a row
+
+// The weight gradients multiply over the samples, so every activation and
+// pre-activation gradient is stored transposed, [feature][sample]: an operand
+// is one 16-byte read.  A wave's own 16 rows pass from layer to layer through
+// `row`, one after the other.
 struct alignas(16) Grad_lds {
     Weights  w;
-    uint16_t x[Chunk * S_feat];
-    uint16_t h[3][Chunk * S_hid];   // post-ReLU activations of the hidden layers
-    uint16_t dz[3][Chunk * S_hid];  // loss gradient at the hidden pre-activations
-    uint16_t dy[Chunk * S_out];     // loss gradient at the outputs
-    float    y[Chunk * S_out];      // outputs
+    uint16_t xt[Feat_pad * S_smp];
+    uint16_t ht[3][Hidden * S_smp];  // post-ReLU activations of the hidden layers
+    uint16_t dzt[3][Hidden * S_smp];  // loss gradient at the hidden pre-activations
+    uint16_t dyt[Num_out * S_smp];    // loss gradient at the outputs
+    alignas(16) uint16_t row[Grad_waves][16 * S_hid];
+    alignas(16) float freq[Num_in * Num_freq];
 };
 static_assert(sizeof(Grad_lds) <= 160 * 1024, "LDS of a workgroup");
-static_assert(offsetof(Grad_lds, x) % 8 == 0 && offsetof(Grad_lds, dy) % 8 == 0 &&
-                  (S_feat * sizeof(uint16_t)) % 4 == 0 && (S_out * sizeof(uint16_t)) % 8 == 0,
-              "packed feature and output-gradient stores are aligned");
+static_assert(offsetof(Grad_lds, xt) % 16 == 0 && offsetof(Grad_lds, dyt) % 16 == 0 &&
+                  (S_smp * sizeof(uint16_t)) % 16 == 0 && (S_hid * sizeof(uint16_t)) % 16 == 0 &&
+                  (S_out * sizeof(uint16_t)) % 16 == 0 && 16 * S_y * sizeof(float) <= 16 * S_hid * sizeof(uint16_t),
+              "16-byte reads are aligned and a wave's outputs fit its rows");
 constexpr int Num_bias = 3 * Hidden + Num_out;  // 224
 
 // Loss gradient at the outputs of lobes q and q + 4 of one sample (row of
@@ -348,21 +325,21 @@ constexpr int Num_bias = 3 * Hidden + Num_out;  // 224
 // hold two lobes each and share the mixture's sums by lane exchange, so
 // every lobe is evaluated once; all 64 lanes must call it.
 struct Lobe_terms {
-    float v, kap, cosk, sa, sb, theta, phi, d;
+    float v, kap, cosk, sa, sb, d;
+    float st, ct, sp, cp;  // sines and cosines of the lobe's angles
+    float em;              // expm1(-2 kappa)
 };
 
 __device__ Lobe_terms lobe_terms(float const* r, float dirx, float diry, float dirz) {
     Lobe_terms t;
     t.sa  = 1.f / (1.f + expf(-r[0]));
     t.sb  = 1.f / (1.f + expf(-r[1]));
-    t.theta = dev::Pi * t.sa;
-    t.phi   = 2.f * dev::Pi * t.sb;
-    float st, ct, sp, cp;
-    sincosf(t.theta, &st, &ct);
-    sincosf(t.phi, &sp, &cp);
-    t.cosk = (st * cp) * dirx + (st * sp) * diry + ct * dirz;
+    sincosf(dev::Pi * t.sa, &t.st, &t.ct);
+    sincosf(2.f * dev::Pi * t.sb, &t.sp, &t.cp);
+    t.cosk = (t.st * t.cp) * dirx + (t.st * t.sp) * diry + t.ct * dirz;
     t.kap  = expf(fminf(fmaxf(r[2], Kappa_lo), Kappa_hi));
-    t.v    = t.kap / (2.f * dev::Pi * -expm1f(-2.f * t.kap)) * expf(t.kap * (t.cosk - 1.f));
+    t.em   = expm1f(-2.f * t.kap);
+    t.v    = t.kap / (2.f * dev::Pi * -t.em) * expf(t.kap * (t.cosk - 1.f));
     t.d    = r[3];
     return t;
 }
@@ -374,15 +351,12 @@ __device__ void lobe_gradient(Lobe_terms const& t, float const* r, float g, floa
     out[3] = g * wk * (t.v - q);
     // kappa: d log v / d kappa = 1/kappa - 2 e^(-2k) / (1 - e^(-2k)) + (cos - 1)
     float const e2  = expf(-2.f * t.kap);
-    float const dlk = 1.f / t.kap - 2.f * e2 / (-expm1f(-2.f * t.kap)) + (t.cosk - 1.f);
+    float const dlk = 1.f / t.kap - 2.f * e2 / (-t.em) + (t.cosk - 1.f);
     bool const  in  = r[2] > Kappa_lo && r[2] < Kappa_hi;
     out[2]          = in ? g * resp * dlk * t.kap : 0.f;
     // direction: d log v / d mu = kappa w
-    float st, ct, sp, cp;
-    sincosf(t.theta, &st, &ct);
-    sincosf(t.phi, &sp, &cp);
-    float const dth = t.kap * ((ct * cp) * dirx + (ct * sp) * diry - st * dirz);
-    float const dph = t.kap * ((-st * sp) * dirx + (st * cp) * diry);
+    float const dth = t.kap * ((t.ct * t.cp) * dirx + (t.ct * t.sp) * diry - t.st * dirz);
+    float const dph = t.kap * ((-t.st * t.sp) * dirx + (t.st * t.cp) * diry);
     out[0]          = g * resp * dth * dev::Pi * t.sa * (1.f - t.sa);
     out[1]          = g * resp * dph * 2.f * dev::Pi * t.sb * (1.f - t.sb);
 }
@@ -410,45 +384,131 @@ __device__ void output_gradients(float const* y, float dirx, float diry, float d
     lobe_gradient(b, y + 4 * (q + 4), g, qm, wb, dirx, diry, dirz, g1);
 }
 
-// dst[16][N] = (src[16][K] W^T) * (act > 0): backward through one layer,
-// W[j][k] = Wt[k][j].  Formed as its transpose like layer(): MFMA A operand
-// A[i][k] = W[16 nt + i][k] = Wt[k][16 nt + i], gathered from 4 rows of Wt;
-// B operand = rows of src; so a lane holds outputs 16 nt + 4q + t of row r,
-// read against the ReLU mask with one 8-byte load and stored with one.
+// A layer's results in a wave, acc[nt][t] = output 16 nt + 4q + t of row r:
+// to the wave's rows (one 8-byte store per tile) and, transposed, to column
+// `sample` of dt.
+template <int N>
+__device__ __forceinline__ void store_rows(float const (&v)[N / 16][4], int r, int q, uint16_t* row,
+                                           int stride, uint16_t* dt, int sample) {
+#pragma unroll
+    for (int nt = 0; nt < N / 16; ++nt) {
+        int const   j0 = nt * 16 + 4 * q;
+        uint2 const pk = make_uint2(pack_bf16(v[nt][0], v[nt][1]), pack_bf16(v[nt][2], v[nt][3]));
+        if (row) {
+            *reinterpret_cast<uint2*>(row + r * stride + j0) = pk;
+        }
+        dt[(j0 + 0) * S_smp + sample] = uint16_t(pk.x);
+        dt[(j0 + 1) * S_smp + sample] = uint16_t(pk.x >> 16);
+        dt[(j0 + 2) * S_smp + sample] = uint16_t(pk.y);
+        dt[(j0 + 3) * S_smp + sample] = uint16_t(pk.y >> 16);
+    }
+}
+
+// ReLU of acc + bias, stored as above; bit 4 nt + t of the result: output
+// 16 nt + 4q + t of row r is positive (as bf16).
+template <int N>
+__device__ __forceinline__ uint32_t store_relu(f32x4 const (&acc)[N / 16], float const* bias, int r,
+                                               int q, uint16_t* row, uint16_t* dt, int sample) {
+    float    v[N / 16][4];
+    uint32_t mask = 0;
+#pragma unroll
+    for (int nt = 0; nt < N / 16; ++nt) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            v[nt][t] = fmaxf(acc[nt][t] + bias[nt * 16 + 4 * q + t], 0.f);
+            mask |= from_bf16(to_bf16(v[nt][t])) > 0.f ? 1u << (4 * nt + t) : 0u;
+        }
+    }
+    store_rows<N>(v, r, q, row, S_hid, dt, sample);
+    return mask;
+}
+
+// acc = W^T A^T over a wave's 16 rows like layer().
 template <int K, int N>
-__device__ void back_layer(uint16_t const* src, int ss, uint16_t const* Wt, int sw,
-                           uint16_t const* act, int sact, uint16_t* dst, int sd) {
-    int const lane = threadIdx.x & 63;
-    int const r    = lane & 15;
-    int const q    = lane >> 4;
-    f32x4     acc[N / 16];
+__device__ __forceinline__ void multiply(uint16_t const* row, int stride, uint16_t const* Wt, int sw,
+                                         int r, int q, f32x4 (&acc)[N / 16]) {
 #pragma unroll
     for (int nt = 0; nt < N / 16; ++nt) {
         acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    static_assert(K % 32 == 0, "depth in steps of 32");
 #pragma unroll
     for (int ks = 0; ks < K / 32; ++ks) {
-        bf16x8 const b = load8(src + r * ss + ks * 32 + 8 * q);
+        bf16x8 const b = load8(row + r * stride + ks * 32 + 8 * q);
 #pragma unroll
         for (int nt = 0; nt < N / 16; ++nt) {
-            acc[nt] = mfma32(gather8(Wt + (ks * 32 + 8 * q) * sw + nt * 16 + r, sw), b, acc[nt]);
+            acc[nt] = mfma32(load8(Wt + (nt * 16 + r) * sw + ks * 32 + 8 * q), b, acc[nt]);
         }
-    }
-#pragma unroll
-    for (int nt = 0; nt < N / 16; ++nt) {
-        int const    j0 = nt * 16 + 4 * q;
-        bf16x4 const m  = load4(act + r * sact + j0);
-        float        v[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            v[t] = from_bf16(uint16_t(m[t])) > 0.f ? acc[nt][t] : 0.f;
-        }
-        *reinterpret_cast<uint2*>(dst + r * sd + j0) =
-            make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
     }
 }
 
+// The operands of a layer's way back, W[16 nt + r][32 ks + 8q ..] =
+// Wt[32 ks + 8q ..][16 nt + r], gathered once per workgroup and kept.
+template <int K, int N>
+struct Back {
+    bf16x8 w[K / 32][N / 16];
+
+    __device__ __forceinline__ void load(uint16_t const* Wt, int sw, int r, int q) {
+#pragma unroll
+        for (int ks = 0; ks < K / 32; ++ks) {
+#pragma unroll
+            for (int nt = 0; nt < N / 16; ++nt) {
+                w[ks][nt] = gather8(Wt + (ks * 32 + 8 * q) * sw + nt * 16 + r, sw);
+            }
+        }
+    }
+
+    // (src[16][K] W^T) * (act > 0), the mask as store_relu gives it
+    __device__ __forceinline__ void run(uint16_t const* src, int stride, uint32_t mask, int r, int q,
+                                        float (&v)[N / 16][4]) const {
+        f32x4 acc[N / 16];
+#pragma unroll
+        for (int nt = 0; nt < N / 16; ++nt) {
+            acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int ks = 0; ks < K / 32; ++ks) {
+            bf16x8 const b = load8(src + r * stride + ks * 32 + 8 * q);
+#pragma unroll
+            for (int nt = 0; nt < N / 16; ++nt) {
+                acc[nt] = mfma32(w[ks][nt], b, acc[nt]);
+            }
+        }
+#pragma unroll
+        for (int nt = 0; nt < N / 16; ++nt) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                v[nt][t] = (mask >> (4 * nt + t)) & 1u ? acc[nt][t] : 0.f;
+            }
+        }
+    }
+};
+
+// Weight gradients of one layer over the chunk's samples: tiles (mt, nt) of
+// act^T dz for mt = mt0, mt0 + step, ..., accumulated in acc.
+template <int Tiles>
+__device__ __forceinline__ void weight_gradients(uint16_t const* act, uint16_t const* dz, int mt0,
+                                                 int step, int nt, int r, int q, f32x4* acc) {
+    bf16x8 b[Chunk / 32];
+#pragma unroll
+    for (int ks = 0; ks < Chunk / 32; ++ks) {
+        // B[k][j] = dz[sample k][j]
+        b[ks] = load8(dz + (nt * 16 + r) * S_smp + ks * 32 + 8 * q);
+    }
+#pragma unroll
+    for (int k = 0; k < Tiles; ++k) {
+#pragma unroll
+        for (int ks = 0; ks < Chunk / 32; ++ks) {
+            // A[i][k] = act[sample k][feature i]
+            bf16x8 const a = load8(act + ((mt0 + step * k) * 16 + r) * S_smp + ks * 32 + 8 * q);
+            acc[k]         = mfma32(a, b[ks], acc[k]);
+        }
+    }
+}
+
+// Bound by the latencies of one wave a SIMD (155 KB of LDS a workgroup).
+// 65 536 samples, 4 chunks a workgroup: 81 us with row-major activations,
+// whose transposed operands took eight 2-byte reads each; 57.6 us with the
+// layout above.
 __global__ void __launch_bounds__(Grad_waves * 64)
     gradient_kernel(uint16_t const* wt, float const* params, float const* freq, float const* x,
                     float const* dirs, float const* weights, uint32_t n, uint32_t const* window,
@@ -463,6 +523,9 @@ __global__ void __launch_bounds__(Grad_waves * 64)
         weights += off;
     }
     load_weights(s.w, wt, params);
+    for (int i = threadIdx.x; i < Num_in * Num_freq; i += blockDim.x) {
+        s.freq[i] = freq[i];
+    }
     __syncthreads();
 
     // thread b < 224 sums the gradient of bias b over the samples, in order
@@ -474,109 +537,158 @@ __global__ void __launch_bounds__(Grad_waves * 64)
     int const q    = lane >> 4;
     float     wacc = 0.f;  // weights of this lane's samples (q == 0), in order
 
+    Back<Num_out, Hidden> back4;
+    Back<Hidden, Hidden>  back3, back2;
+    back4.load(s.w.w4, S_hid, r, q);
+    back3.load(s.w.w3, S_hid, r, q);
+    back2.load(s.w.w2, S_hid, r, q);
+
     f32x4 acc[Tiles_per_wave];
 #pragma unroll
     for (int k = 0; k < Tiles_per_wave; ++k) {
         acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
+    uint16_t* const R      = s.row[wave];
+    float* const    Y      = reinterpret_cast<float*>(R);
+    int const       sample = wave * 16 + r;  // of the chunk
+
     uint32_t const chunks = (n + Chunk - 1) / Chunk;
     for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {  // block-uniform
-        uint32_t const row0 = c * Chunk + wave * 16;
-        uint16_t*      X    = s.x + wave * 16 * S_feat;
-        uint16_t*      H1   = s.h[0] + wave * 16 * S_hid;
-        uint16_t*      H2   = s.h[1] + wave * 16 * S_hid;
-        uint16_t*      H3   = s.h[2] + wave * 16 * S_hid;
-        uint16_t*      DZ1  = s.dz[0] + wave * 16 * S_hid;
-        uint16_t*      DZ2  = s.dz[1] + wave * 16 * S_hid;
-        uint16_t*      DZ3  = s.dz[2] + wave * 16 * S_hid;
-        uint16_t*      DY   = s.dy + wave * 16 * S_out;
-        float*         Y    = s.y + wave * 16 * S_out;
+        uint32_t const row  = c * Chunk + sample;
+        bool const     live = row < n;
+        // unnormalized weights: the reduction divides by the batch's weight sum
+        float const tw  = live ? weights[row] : 0.f;
+        float const dx  = live ? dirs[3 * size_t(row) + 0] : 0.f;
+        float const dyv = live ? dirs[3 * size_t(row) + 1] : 0.f;
+        float const dz  = live ? dirs[3 * size_t(row) + 2] : 1.f;
 
-        features(x, freq, row0, n, X);
+        uint32_t mask1, mask2, mask3;
+        {
+            // Layer 1 with its features formed in registers: the operand of
+            // lane (r, q) at depth step ks is features k0 .. k0 + 7 of row r,
+            // sin / cos of pi (freq[i][j] x_i), the product rounded to fp32;
+            // zero past the 216 features and for rows past n.  sin(pi f) =
+            // sin(2 pi (f / 2)): the hardware sine of the fraction of f / 2
+            // turns (f / 2 and its fraction are exact).
+            f32x4 a1[Hidden / 16];
+#pragma unroll
+            for (int nt = 0; nt < Hidden / 16; ++nt) {
+                a1[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            static_assert(Feat_pad % 32 == 0 && 24 % 8 == 0, "eight features of one input per lane");
+#pragma unroll
+            for (int ks = 0; ks < Feat_pad / 32; ++ks) {
+                int const k0   = ks * 32 + 8 * q;
+                uint32_t  w[4] = {0u, 0u, 0u, 0u};
+                if (k0 < Num_feat && live) {
+                    int const   i  = k0 / 24;
+                    int const   j0 = (k0 % 24) / 2;
+                    float const v  = x[size_t(row) * Num_in + i];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        float const f   = s.freq[i * Num_freq + j0 + u] * v;
+                        float const h   = 0.5f * f;
+                        float const rev = h - floorf(h);
+                        w[u] = pack_bf16(__builtin_amdgcn_sinf(rev), __builtin_amdgcn_cosf(rev));
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    s.xt[(k0 + 2 * u) * S_smp + sample]     = uint16_t(w[u]);
+                    s.xt[(k0 + 2 * u + 1) * S_smp + sample] = uint16_t(w[u] >> 16);
+                }
+                bf16x8 const b = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+#pragma unroll
+                for (int nt = 0; nt < Hidden / 16; ++nt) {
+                    a1[nt] = mfma32(load8(s.w.w1 + (nt * 16 + r) * S_feat + k0), b, a1[nt]);
+                }
+            }
+            mask1 = store_relu<Hidden>(a1, s.w.b, r, q, R, s.ht[0], sample);
+        }
         wave_sync();
-        layer<Feat_pad, Hidden, Mode_relu>(X, S_feat, s.w.w1, S_feat, s.w.b, H1, S_hid, nullptr, 0);
+        f32x4 a[Hidden / 16];
+        multiply<Hidden, Hidden>(R, S_hid, s.w.w2, S_hid, r, q, a);
+        wave_sync();  // the rows are read before they are written
+        mask2 = store_relu<Hidden>(a, s.w.b + Hidden, r, q, R, s.ht[1], sample);
         wave_sync();
-        layer<Hidden, Hidden, Mode_relu>(H1, S_hid, s.w.w2, S_hid, s.w.b + Hidden, H2, S_hid, nullptr, 0);
+        multiply<Hidden, Hidden>(R, S_hid, s.w.w3, S_hid, r, q, a);
         wave_sync();
-        layer<Hidden, Hidden, Mode_relu>(H2, S_hid, s.w.w3, S_hid, s.w.b + 2 * Hidden, H3, S_hid, nullptr, 0);
+        mask3 = store_relu<Hidden>(a, s.w.b + 2 * Hidden, r, q, R, s.ht[2], sample);
         wave_sync();
-        layer<Hidden, Num_out, Mode_f32>(H3, S_hid, s.w.w4, S_hid, s.w.b + 3 * Hidden, nullptr, 0, Y, S_out);
+        f32x4 ay[Num_out / 16];
+        multiply<Hidden, Num_out>(R, S_hid, s.w.w4, S_hid, r, q, ay);
+        wave_sync();
+#pragma unroll
+        for (int nt = 0; nt < Num_out / 16; ++nt) {
+            int const j0 = nt * 16 + 4 * q;
+            float     o[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                o[t] = ay[nt][t] + s.w.b[3 * Hidden + j0 + t];
+            }
+            *reinterpret_cast<float4*>(Y + r * S_y + j0) = make_float4(o[0], o[1], o[2], o[3]);
+        }
         wave_sync();
 
         // output gradients: lane handles sample r, lobes q and q + 4
         {
-            uint32_t const row = row0 + r;
-            float          g0[4];
-            float          g1[4];
-            // unnormalized weights: the reduction divides by the batch's weight sum
-            float const tw  = row < n ? weights[row] : 0.f;
-            float const dx  = row < n ? dirs[3 * size_t(row) + 0] : 0.f;
-            float const dyv = row < n ? dirs[3 * size_t(row) + 1] : 0.f;
-            float const dz  = row < n ? dirs[3 * size_t(row) + 2] : 1.f;
+            float g[2][4];
             if (0 == q) {
                 wacc += tw;
             }
-            output_gradients(Y + r * S_out, dx, dyv, dz, tw, q, g0, g1);
-            wave_sync();  // Y is read by all lanes before DY and DZ1 are written
-            // four consecutive outputs per store (offsets are multiples of 4 elements)
-            *reinterpret_cast<uint2*>(DY + r * S_out + 4 * q) =
-                make_uint2(pack_bf16(g0[0], g0[1]), pack_bf16(g0[2], g0[3]));
-            *reinterpret_cast<uint2*>(DY + r * S_out + 4 * (q + 4)) =
-                make_uint2(pack_bf16(g1[0], g1[1]), pack_bf16(g1[2], g1[3]));
+            output_gradients(Y + r * S_y, dx, dyv, dz, tw, q, g[0], g[1]);
+            wave_sync();  // the outputs are read by all lanes before the rows are written
+            store_rows<Num_out>(g, r, q, R, S_out, s.dyt, sample);
         }
         wave_sync();
-        back_layer<Num_out, Hidden>(DY, S_out, s.w.w4, S_hid, H3, S_hid, DZ3, S_hid);
+        float v[Hidden / 16][4];
+        back4.run(R, S_out, mask3, r, q, v);
         wave_sync();
-        back_layer<Hidden, Hidden>(DZ3, S_hid, s.w.w3, S_hid, H2, S_hid, DZ2, S_hid);
+        store_rows<Hidden>(v, r, q, R, S_hid, s.dzt[2], sample);
         wave_sync();
-        back_layer<Hidden, Hidden>(DZ2, S_hid, s.w.w2, S_hid, H1, S_hid, DZ1, S_hid);
+        back3.run(R, S_hid, mask2, r, q, v);
+        wave_sync();
+        store_rows<Hidden>(v, r, q, R, S_hid, s.dzt[1], sample);
+        wave_sync();
+        back2.run(R, S_hid, mask1, r, q, v);
+        store_rows<Hidden>(v, r, q, nullptr, 0, s.dzt[0], sample);
         __syncthreads();
 
-        // bias gradients: column sums over the chunk's samples
+        // bias gradients: sums over the chunk's samples
         if (int(threadIdx.x) < Num_bias) {
             int const       b   = threadIdx.x;
-            uint16_t const* src = b < 3 * Hidden ? s.dz[b / Hidden] + b % Hidden : s.dy + (b - 3 * Hidden);
-            int const       st  = b < 3 * Hidden ? S_hid : S_out;
-            for (int k = 0; k < Chunk; ++k) {
-                bias_acc += from_bf16(src[k * st]);
+            uint16_t const* src = b < 3 * Hidden ? s.dzt[b / Hidden] + (b % Hidden) * S_smp
+                                                 : s.dyt + (b - 3 * Hidden) * S_smp;
+#pragma unroll
+            for (int k = 0; k < Chunk; k += 8) {
+                uint4 const    pk   = *reinterpret_cast<uint4 const*>(src + k);
+                uint32_t const w[4] = {pk.x, pk.y, pk.z, pk.w};
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    bias_acc += from_bf16(uint16_t(w[u]));
+                    bias_acc += from_bf16(uint16_t(w[u] >> 16));
+                }
             }
         }
 
-        // weight gradients over the chunk's 64 samples: dW = act^T dz
-#pragma unroll
-        for (int k = 0; k < Tiles_per_wave; ++k) {
-            int const tile = wave + Grad_waves * k;
-            uint16_t const* act;
-            uint16_t const* dz;
-            int sa, sd, mt, nt;
-            if (tile < 56) {
-                act = s.x, sa = S_feat, dz = s.dz[0], sd = S_hid, mt = tile / 4, nt = tile % 4;
-            } else if (tile < 72) {
-                act = s.h[0], sa = S_hid, dz = s.dz[1], sd = S_hid, mt = (tile - 56) / 4, nt = (tile - 56) % 4;
-            } else if (tile < 88) {
-                act = s.h[1], sa = S_hid, dz = s.dz[2], sd = S_hid, mt = (tile - 72) / 4, nt = (tile - 72) % 4;
-            } else {
-                act = s.h[2], sa = S_hid, dz = s.dy, sd = S_out, mt = (tile - 88) / 2, nt = (tile - 88) % 2;
-            }
-#pragma unroll
-            for (int ks = 0; ks < Chunk / 32; ++ks) {
-                // A[i][k] = act[sample k][feature i]; B[k][j] = dz[sample k][j]
-                bf16x8 const a = gather8(act + (ks * 32 + 8 * q) * sa + mt * 16 + r, sa);
-                bf16x8 const b = gather8(dz + (ks * 32 + 8 * q) * sd + nt * 16 + r, sd);
-                acc[k]         = mfma32(a, b, acc[k]);
-            }
-        }
+        // weight gradients over the chunk's 64 samples: dW = act^T dz, tile
+        // wave + 4 k of the 56 + 16 + 16 + 8
+        weight_gradients<14>(s.xt, s.dzt[0], 0, 1, wave, r, q, acc);
+        weight_gradients<4>(s.ht[0], s.dzt[1], 0, 1, wave, r, q, acc + 14);
+        weight_gradients<4>(s.ht[1], s.dzt[2], 0, 1, wave, r, q, acc + 18);
+        weight_gradients<2>(s.ht[2], s.dyt, wave / 2, 2, wave % 2, r, q, acc + 22);
         __syncthreads();
     }
 
-    // the workgroup's weight sum, lanes in a fixed order (reusing s.y)
-    s.y[threadIdx.x] = wacc;
+    // the workgroup's weight sum, lanes in a fixed order (reusing the rows)
+    float* const sums = reinterpret_cast<float*>(s.row);
+    sums[threadIdx.x] = wacc;
     __syncthreads();
     if (0 == threadIdx.x) {
         float t = 0.f;
         for (int k = 0; k < Grad_waves * 64; ++k) {
-            t += s.y[k];
+            t += sums[k];
         }
         wsum[blockIdx.x] = t;
     }
