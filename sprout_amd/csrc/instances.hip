@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(Block) trace_instances(Tlas_view t, mi_ray con
 // pushed as {its node word, its box entry distance} and the near one taken.
 // A popped child is skipped when its entry distance exceeds the current
 // max_t, which is exactly the reference's box test of it at that max_t
-// (slab_entry).  A node word packs data (< 2^22), axis and count, so popped
+// (slab_lean).  A node word packs data (< 2^22), axis and count, so popped
 // children need no node fetch.  The mesh walk runs above a sentinel word on
 // the same stack.  The first Lds_entries entries of a lane live in LDS, the
 // rest in a per-thread global area.

@@ -13,7 +13,7 @@
 //          The edge vectors are the same rounded differences the reference
 //          computes per test, so the intersection arithmetic is unchanged.
 //
-// Two loops, both bit-identical to the reference in result:
+// Three loops, all bit-identical to the reference in result:
 //   * trace_pairs: one thread per ray over a persistent grid.  At an inner
 //     node both children are tested from one 64-byte fetch; the far child
 //     (by the sign of inv_dir on the node's axis, as the reference) is pushed
@@ -24,8 +24,10 @@
 //     descend near), counting node fetches and triangle tests per ray; this
 //     gives the algorithmic bytes per ray.
 //   * trace_refill(_packed): persistent waves that refill idle lanes with new
-//     rays; the packed variant's stack entries carry the far child's node
-//     word and box entry distance, so a pop needs no node fetch.
+//     rays (claims.hpp); the packed variant's stack entries carry the far
+//     child's node word and box entry distance, so a pop needs no node fetch,
+//     and its waves take one kind of step a turn, the kind most lanes wait
+//     for.
 // The traversal stack lives in LDS (Lds_entries per lane, laid out
 // entry-major so a wave's 64 lanes hit 64 different banks) and spills to a
 // per-thread global area beyond that, sized from the tree's depth.
@@ -530,7 +532,7 @@ __global__ void trace_refill(Launch p) {
 // count, so a popped child continues without fetching its node again, and a
 // popped child whose entry distance exceeds the current max_t is skipped: the
 // reference's box test of that child at this max_t is exactly max_t >= tmin
-// (slab_entry), the rest of it held when the child was pushed.
+// (slab_lean), the rest of it held when the child was pushed.
 constexpr uint32_t Packed_data_bits = 22;
 
 __device__ __forceinline__ uint32_t pack_node(uint32_t data, uint32_t meta) {
