@@ -154,43 +154,60 @@ __device__ inline bool intersect_inside(V3 lo, V3 hi, Tray const& r, float& hit_
     return max_out >= r.min_t && r.min_t >= min_out && r.max_t >= min_out && max_out >= min_out;
 }
 
-// Gridtree::intersect: clips r.max_t to the leaf cell around r.point(min_t).
-// The tree's leaves are laid out per block of its smallest leaf size, so a
-// cell is one load away instead of a chain of up to four.
-__device__ inline bool gridtree_intersect(Medium_view const& m, Tray& r, Medium_cm& cm) {
+// The leaf around a point in texture space: its level (| Leaf_empty) and
+// coefficients, or Leaf_outside.  The tree's leaves are laid out per block of
+// its smallest leaf size, so a cell is one load away instead of a chain of up
+// to four.
+inline constexpr uint32_t Leaf_outside = 0xFFu;
+
+struct Leaf {
+    uint32_t  level;
+    Medium_cm cm;
+};
+
+__device__ __forceinline__ Leaf fetch_leaf(Medium_view const& m, V3 p) {
+    int32_t const cx = int32_t(float(m.dims[0]) * p.x);
+    int32_t const cy = int32_t(float(m.dims[1]) * p.y);
+    int32_t const cz = int32_t(float(m.dims[2]) * p.z);
+    Leaf          l;
+    l.level = Leaf_outside;
+    if (uint32_t(cx >> Log2_cell_dim) < m.num_cells[0] && uint32_t(cy >> Log2_cell_dim) < m.num_cells[1] &&
+        uint32_t(cz >> Log2_cell_dim) < m.num_cells[2]) {
+        uint32_t const bx    = m.num_cells[0] << (Log2_cell_dim - Log2_block_dim);
+        uint32_t const by    = m.num_cells[1] << (Log2_cell_dim - Log2_block_dim);
+        size_t const   block = (size_t(cz >> Log2_block_dim) * by + uint32_t(cy >> Log2_block_dim)) * bx +
+                             uint32_t(cx >> Log2_block_dim);
+        l.level = m.levels[block];
+        l.cm    = m.leaves[block];
+    }
+    return l;
+}
+
+// Gridtree::intersect: clips r.max_t to the leaf cell around r.point(min_t),
+// whose level is given; false outside of the tree and where the ray misses
+// the cell.
+__device__ inline bool gridtree_intersect(Medium_view const& m, Tray& r, uint32_t level) {
+    if (Leaf_outside == level) {
+        return false;
+    }
     V3 const      p  = r.point(r.min_t);
     int32_t const cx = int32_t(float(m.dims[0]) * p.x);
     int32_t const cy = int32_t(float(m.dims[1]) * p.y);
     int32_t const cz = int32_t(float(m.dims[2]) * p.z);
-    int32_t const vx = cx >> Log2_cell_dim;
-    int32_t const vy = cy >> Log2_cell_dim;
-    int32_t const vz = cz >> Log2_cell_dim;
-    if (uint32_t(vx) >= m.num_cells[0] || uint32_t(vy) >= m.num_cells[1] ||
-        uint32_t(vz) >= m.num_cells[2]) {
-        return false;
-    }
-    uint32_t const bx    = m.num_cells[0] << (Log2_cell_dim - Log2_block_dim);
-    uint32_t const by    = m.num_cells[1] << (Log2_cell_dim - Log2_block_dim);
-    size_t const   block = (size_t(cz >> Log2_block_dim) * by + uint32_t(cy >> Log2_block_dim)) * bx +
-                         uint32_t(cx >> Log2_block_dim);
-    uint32_t const level = m.levels[block];
-    Medium_cm const leaf = m.leaves[block];
     int32_t const  size  = Cell_dim >> (level & 3u);
     int32_t const  b0[3] = {cx & -size, cy & -size, cz & -size};
     int32_t const  b1[3] = {b0[0] + size, b0[1] + size, b0[2] + size};
     V3 const lo = v3(float(b0[0]) * m.inv_dims[0], float(b0[1]) * m.inv_dims[1], float(b0[2]) * m.inv_dims[2]);
     V3 const hi = v3(float(b1[0]) * m.inv_dims[0], float(b1[1]) * m.inv_dims[1], float(b1[2]) * m.inv_dims[2]);
     float hit_t;
-    if (intersect_inside(lo, hi, r, hit_t)) {
-        if (r.max_t > hit_t) {
-            r.max_t = hit_t;
-        }
-    } else {
+    if (!intersect_inside(lo, hi, r, hit_t)) {
         r.max_t = r.min_t;
         return false;
     }
-    cm = leaf;
-    return 0 == (level & Leaf_empty);
+    if (r.max_t > hit_t) {
+        r.max_t = hit_t;
+    }
+    return true;
 }
 
 // van_de_hulst(g, gs) with gs lerped towards 0 over the range
@@ -373,6 +390,7 @@ struct Walk {
     float          srs;
     float          w[NC];    // multiplies the throughput
     bool           nearest;
+    Leaf           next;     // of the cell to enter next, fetched a step ahead
 
     __device__ __forceinline__ uint32_t start(Medium_view const& m, V3 o, V3 d, float t0, float t1,
                                               uint32_t depth, bool nearest_) {
@@ -380,6 +398,7 @@ struct Walk {
         end     = t1;
         srs     = similarity_scale(m.g, depth);
         nearest = nearest_;
+        next    = fetch_leaf(m, r.point(r.min_t));
         for (int c = 0; c < NC; ++c) {
             w[c] = 1.f;
         }
@@ -394,10 +413,13 @@ struct Walk {
 
     template <typename Rng>
     __device__ __forceinline__ uint32_t enter_cell(Medium_view const& m, Rng& rng) {
-        Medium_cm cm;
-        if (!gridtree_intersect(m, r, cm)) {
+        Leaf const leaf = next;
+        bool const hit  = gridtree_intersect(m, r, leaf.level);
+        next            = fetch_leaf(m, r.point(offset_f(r.max_t)));
+        if (!hit || (leaf.level & Leaf_empty)) {
             return leave_cell();
         }
+        Medium_cm cm = leaf.cm;
         cm.minorant_mu_s *= srs;
         cm.majorant_mu_s *= srs;
         mt = cm.majorant_mu_a + cm.majorant_mu_s;
