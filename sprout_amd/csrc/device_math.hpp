@@ -84,17 +84,30 @@ __device__ __forceinline__ bool slab(float4 lo, float4 hi, F3 o, F3 inv, float m
     return (tmax >= min_t) & (max_t >= tmin) & (tmax >= tmin);
 }
 
+// max / min of two products, NaN if either is (v_maximum3_f32, v_minimum3_f32)
+__device__ __forceinline__ float either_max(float a, float b) {
+    return __builtin_elementwise_maximum(a, b);
+}
+
+__device__ __forceinline__ float either_min(float a, float b) {
+    return __builtin_elementwise_minimum(a, b);
+}
+
 // slab with the box's entry distance tmin: while the ray's min_t and
 // direction stay, the test at a smaller max_t' is exactly max_t' >= tmin
 // (the other two terms do not involve max_t).
-// It goes without the per-coordinate NaN filters, for boxes without NaN
-// coordinates.  A coordinate product is NaN then only where the ray's
-// inverse direction or origin is (both ends of the axis alike, dropped by
-// min / max as the filter drops them; with all three axes gone the negated
-// comparisons below admit the box as the filtered infinities do), or
-// where an infinite origin meets an infinite bound, a ray no triangle
-// accepts.  24 operations a box instead of 36; tmin may be NaN (all axes
-// gone) and compares as -infinity through !(max_t < tmin).
+// The same test without slab's per-coordinate filters, for every box and ray
+// whose min_t and max_t are numbers.  The filters make an axis with a NaN
+// product unbounded, [-inf, inf], also where only one end is NaN: a ray that
+// starts on one of the box's planes with an infinite inverse direction there
+// (reciprocal_lane of components from 2.9e-39 to 5.4e-20 in size, whose r * r
+// overflows) has 0 * inf at that end.  Here such an axis is NaN as a whole and
+// the outer fminf / fmaxf drop it; with all three gone tmax and tmin are NaN,
+// which the negated comparisons admit as they admit the infinities.  24
+// operations a box instead of 36: 4.2 M bounce rays over 1.41 M triangles 1708
+// us with the filters and 1644 without, 480 k occlusion rays 245 and 224 us,
+// 1 M rays into 64 instances 687 and 666 us.  A NaN tmin compares as
+// -infinity through !(max_t < tmin).
 __device__ __forceinline__ bool slab_lean(float4 lo, float4 hi, F3 o, F3 inv, float min_t,
                                           float max_t, float& tmin_out) {
     float const l1x = (lo.x - o.x) * inv.x;
@@ -104,8 +117,8 @@ __device__ __forceinline__ bool slab_lean(float4 lo, float4 hi, F3 o, F3 inv, fl
     float const l2y = (hi.y - o.y) * inv.y;
     float const l2z = (hi.z - o.z) * inv.z;
 
-    float const tmax = fminf(fminf(fmaxf(l1x, l2x), fmaxf(l1y, l2y)), fmaxf(l1z, l2z));
-    float const tmin = fmaxf(fmaxf(fminf(l1x, l2x), fminf(l1y, l2y)), fminf(l1z, l2z));
+    float const tmax = fminf(fminf(either_max(l1x, l2x), either_max(l1y, l2y)), either_max(l1z, l2z));
+    float const tmin = fmaxf(fmaxf(either_min(l1x, l2x), either_min(l1y, l2y)), either_min(l1z, l2z));
     tmin_out         = tmin;
     return !(tmax < min_t) & !(max_t < tmin) & !(tmax < tmin);
 }

@@ -1,7 +1,8 @@
 """The default traversal over the launch sizes and ray forms where its rules
 change: slices of fewer than 64 rays a wave, the last slice, the first
-claimed ray; rays with zero, NaN or infinite components; trees whose bounds
-are not finite.  Every word must equal the reference-order loop's
+claimed ray; rays with zero, NaN or infinite components, and rays that start
+on a node's bound with an infinite inverse direction there, also through
+instances; trees whose bounds are not finite.  Every word must equal the reference-order loop's
 (mi_trace_counts), which the other tests pin to the oracle."""
 
 import numpy as np
@@ -41,13 +42,13 @@ def rays_of(n, seed=1):
     return r
 
 
-def agree(gpu, tree, rays):
+def agree(gpu, tree, rays, kernels=(3, 4)):
     import torch
 
     d = torch.from_numpy(rays).cuda()
     for any_hit in (False, True):
         want, _ = tree.counts(d, any_hit=any_hit)
-        for kernel in (3, 4):
+        for kernel in kernels:
             gpu.set_trace_config(kernel=kernel)
             got = tree.intersect_p(d) if any_hit else tree.intersect(d)
             torch.cuda.synchronize()
@@ -123,3 +124,83 @@ def test_vertex_not_finite(gpu, mesh):
     tree = gpu.Builder_SAH().build(torch.from_numpy(p).cuda(),
                                    torch.from_numpy(idx.view(np.int32)).cuda())
     agree(gpu, tree, rays_of(4096, 6))
+
+
+def rays_on_planes(n, seed, values):
+    """rays along the planes x, y or z = one of values (and edges, where two
+    axes are chosen), with direction components there whose inverse is
+    infinite (1e-20, 1e-30, 3.7e-33, 5.4e-20), zero's NaN or finite"""
+    r = rays_of(n, seed)
+    rng = np.random.default_rng(seed + 1)
+    flat = np.array([1e-20, -1e-20, 1e-30, -1e-30, 3.7e-33, -3.7e-33, 5.4e-20, -5.4e-20, 0.0, 6e-17], np.float32)
+    for i in range(n):
+        for c in rng.choice(3, rng.integers(1, 3), replace=False):
+            v = values[c]
+            r[i, c] = v[rng.integers(len(v))]
+            r[i, 4 + c] = flat[rng.integers(len(flat))]
+    return r
+
+
+def grid_mesh(n):
+    """a flat n x n grid at z = 0 whose lines are bounds of its nodes"""
+    x, y = np.meshgrid(np.arange(n + 1), np.arange(n + 1), indexing="ij")
+    pos = np.stack([x, y, 0.25 * ((x + y) % 2)], -1).reshape(-1, 3).astype(np.float32) / n - np.float32(0.5)
+    a = (np.arange(n)[:, None] * (n + 1) + np.arange(n)[None, :]).reshape(-1)
+    idx = np.concatenate([np.stack([a, a + n + 1, a + n + 2], 1), np.stack([a, a + n + 2, a + 1], 1)])
+    return pos, idx.astype(np.uint32)
+
+
+@pytest.mark.parametrize("which", ["grid", "sphere"])
+def test_origins_on_bounds(gpu, mesh, which):
+    pos, idx, otree = mesh
+    if which == "grid":
+        pos, idx = grid_mesh(16)
+        otree = O.build(pos, idx)
+    tree = gpu.upload(otree.nodes, otree.slots, pos, idx)
+    planes = [np.concatenate([otree.nodes["lo"][:, c], otree.nodes["hi"][:, c]]) for c in range(3)]
+    rays = rays_on_planes(20000, 11, planes)
+    agree(gpu, tree, rays, kernels=(2, 3))
+    # and against the oracle's own walk
+    import torch
+
+    d = torch.from_numpy(rays).cuda()
+    got = tree.intersect(d).cpu().numpy().view(np.uint32)
+    want = O.trace(otree, pos, idx, rays)
+    assert np.array_equal(got, want)
+    assert (want[:, 3] != 0xFFFFFFFF).mean() > 0.05
+    # the compressed boxes of kernel 4 are larger: it may also find a hit in a
+    # box that a ray along its plane misses by a rounding, and loses none
+    gpu.set_trace_config(kernel=4)
+    wide = tree.intersect(d).cpu().numpy().view(np.uint32)
+    gpu.set_trace_config(kernel=3)
+    more = np.any(wide != want, axis=1)
+    nearest = O.brute_force(pos, idx, rays)
+    assert (wide[more, 0].view(np.float32) <= want[more, 0].view(np.float32)).all()
+    assert (wide[more, 0].view(np.float32) >= nearest[more, 0].view(np.float32)).all()
+    assert more.mean() < 0.05
+
+
+def test_origins_on_bounds_of_instances(gpu):
+    """the instances are moved by whole grid cells, so that a world ray on a
+    plane of the grid is on one in object space too"""
+    import torch
+
+    from sprout_amd import instances
+
+    pos, idx = grid_mesh(8)
+    tree = gpu.Builder_SAH().build(torch.from_numpy(pos).cuda(), torch.from_numpy(idx.view(np.int32)).cuda())
+    n = 9
+    o2w = np.tile(np.eye(4, dtype=np.float32), (n, 1, 1))
+    o2w[:, 3, :3] = [(i % 3 - 1, i // 3 - 1, 0.25 * (i % 2)) for i in range(n)]
+    w2o = np.linalg.inv(o2w.astype(np.float64)).astype(np.float32)
+    inst = instances.Instances([tree] * n, w2o, o2w)
+    ref = O.Instances([(pos, idx, O.build(pos, idx))], np.zeros(n, np.uint32), w2o, o2w)
+    lines = [np.arange(-12, 13, dtype=np.float32) / 8] * 2 + [np.arange(-4, 5, dtype=np.float32) / 8]
+    rays = rays_on_planes(20000, 21, lines)
+    d = torch.from_numpy(rays).cuda()
+    for any_hit in (False, True):
+        got = (inst.intersect_p(d) if any_hit else inst.intersect(d)).cpu().numpy().view(np.uint32)
+        want = ref.trace(rays, any_hit=any_hit)
+        assert np.array_equal(got if any_hit else got[:, :5], want), any_hit
+    assert want.mean() > 0.05
+    inst.release()
