@@ -708,9 +708,9 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
 
     // the two-word stack traversal: every tree's node words must pack, and
     // the deepest stack beyond its LDS part spills to a per-thread area
-    bool packs = !out.tree.nan_bounds && out.tree.num_nodes < (1u << Data_bits) && out.tree.num_slots < (1u << Data_bits);
+    bool packs = out.tree.num_nodes < (1u << Data_bits) && out.tree.num_slots < (1u << Data_bits);
     for (uint32_t k = 0; k < num_meshes; ++k) {
-        packs = packs && !meshes[k]->nan_bounds && meshes[k]->num_nodes < (1u << Data_bits) &&
+        packs = packs && meshes[k]->num_nodes < (1u << Data_bits) &&
                 meshes[k]->num_slots < (1u << Data_bits);
     }
     if (packs) {

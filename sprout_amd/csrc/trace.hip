@@ -946,14 +946,15 @@ namespace {
 
 // The two-word stack holds node words of trees below 2^22 nodes and slots.
 bool packable(DeviceBvh const& bvh) {
-    return !bvh.nan_bounds && bvh.num_nodes < (1u << Packed_data_bits) && bvh.num_slots < (1u << Packed_data_bits);
+    return bvh.num_nodes < (1u << Packed_data_bits) && bvh.num_slots < (1u << Packed_data_bits);
 }
 
 // The compressed pairs of kernel 4 (made once per tree): a grid of 65 535
 // steps per axis over the root box, its scale grown until the last step
-// reaches the box's upper corner.
+// reaches the box's upper corner.  A bound that is not finite has no place on
+// a grid: kernel 3 serves such a tree.
 int32_t ensure_quantized(DeviceBvh const& bvh, hipStream_t stream) {
-    if (bvh.qpairs || bvh.qfailed || bvh.num_nodes < 3) {
+    if (bvh.qpairs || bvh.qfailed || bvh.nan_bounds || bvh.num_nodes < 3) {
         return MI_OK;
     }
     uint32_t const num_pairs = (bvh.num_nodes - 1) / 2;

@@ -126,6 +126,40 @@ def test_vertex_not_finite(gpu, mesh):
     agree(gpu, tree, rays_of(4096, 6))
 
 
+def test_hits_beside_a_vertex_not_finite(gpu, mesh):
+    """the other triangles of such a mesh are hit as if it were not there,
+    alone and instanced"""
+    import torch
+
+    from sprout_amd import instances
+
+    pos, idx, _ = mesh
+    p = pos.copy()
+    p[7, 1] = p[300, 0] = np.nan
+    tree = gpu.Builder_SAH().build(torch.from_numpy(p).cuda(),
+                                   torch.from_numpy(idx.view(np.int32)).cuda())
+    rays = rays_of(4096, 8)
+    d = torch.from_numpy(rays).cuda()
+    bad = ~np.isfinite(p[idx].reshape(len(idx), -1)).all(axis=1)
+    q = p.copy()
+    q[~np.isfinite(q)] = 0.0
+    want = O.brute_force(q, idx[~bad], rays)
+    ids = np.flatnonzero(~bad).astype(np.uint32)
+    hit = want[:, 3] != 0xFFFFFFFF
+    want[hit, 3] = ids[want[hit, 3]]
+    assert bad.any() and hit.mean() > 0.25
+    for kernel in (2, 3, 4):
+        gpu.set_trace_config(kernel=kernel)
+        got = tree.intersect(d).cpu().numpy().view(np.uint32)
+        gpu.set_trace_config(kernel=3)
+        assert np.array_equal(got, want), kernel
+    eye = np.eye(4, dtype=np.float32)[None]
+    inst = instances.Instances([tree], eye, eye)
+    got = inst.intersect(d).cpu().numpy().view(np.uint32)
+    assert np.array_equal(got[:, :4], want)
+    inst.release()
+
+
 def rays_on_planes(n, seed, values):
     """rays along the planes x, y or z = one of values (and edges, where two
     axes are chosen), with direction components there whose inverse is
