@@ -99,6 +99,11 @@ int32_t fail(int32_t status, char const* fmt, ...) {
     va_start(args, fmt);
     std::vsnprintf(last_error, sizeof(last_error), fmt, args);
     va_end(args);
+    if (MI_ERR_HIP == status) {
+        // reported: the runtime keeps it too, where the next check of a
+        // launch, here or elsewhere in the program, would take it for its own
+        (void)hipGetLastError();
+    }
     return status;
 }
 

@@ -5,6 +5,8 @@ here touches a GPU."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -113,3 +115,32 @@ def test_generators_reject_bad_arguments():
         pos = np.zeros((3, 3), np.float32)
         idx = np.zeros((1, 3), np.uint32)
         scenes.bounce_rays(rays, hits, pos, idx, 4)
+
+
+RUNTIME_STUB = """
+static int pending;
+int hipGetDeviceCount(int* n) { *n = 0; return pending = 100; }
+int hipGetLastError(void) { int e = pending; pending = 0; return e; }
+int stub_pending(void) { return pending; }
+"""
+
+FAILED_CALL = """
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+assert lib.mi_init(0) == -3, "no device"
+sys.exit(stub.stub_pending())
+"""
+
+
+def test_a_failed_call_leaves_no_error_behind(tmp_path):
+    """the HIP runtime keeps a failed call's error for the thread's next check
+    of a launch: one that the library has reported must not be found there, by
+    the library's next call or by another user of the runtime (here the
+    runtime's calls are a stub's, which has no device)"""
+    stub = tmp_path / "stub.so"
+    (tmp_path / "stub.c").write_text(RUNTIME_STUB)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(stub), str(tmp_path / "stub.c")], check=True)
+    r = subprocess.run([sys.executable, "-c", FAILED_CALL, str(stub), _lib.load()._name],
+                       capture_output=True, text=True, timeout=120)
+    assert 0 == r.returncode, (r.returncode, r.stderr)
