@@ -43,8 +43,11 @@
 // MI_ERR_UNSPLITTABLE (the reference logs and leaves the node
 // uninitialized); a grid node whose box has zero extent gets no slice
 // candidates (the reference converts NaN to an integer step count).  Bounds
-// equal up to the sign of zero may differ in that sign, and a NaN bound does
-// not enter a node's box.
+// equal up to the sign of zero may differ in that sign.  A triangle with a
+// vertex that is not finite is in the tree with the box of its finite
+// coordinates (make_refs): no ray hits it, and NaN or infinite bounds give
+// NaN costs, on which nodes split until memory or the levels run out, or drop
+// the bounds of the triangles beside it.
 
 #include "bvh_build.hpp"
 #include "device_math.hpp"
@@ -74,7 +77,7 @@ constexpr float Flt_max = 3.40282347e+38f;
 constexpr uint32_t Err_unsplittable = 1;
 constexpr uint32_t Err_index        = 2;
 constexpr uint32_t Err_layout       = 8;
-constexpr uint32_t Not_finite       = 16;  // no error: a vertex is not finite
+constexpr uint32_t Not_finite       = 16;  // no error: an instance's box is not finite
 constexpr uint32_t Err_capacity     = 32;  // a list or buffer is full: the host starts over with more
 constexpr uint32_t Err_stop         = Err_unsplittable | Err_index | Err_capacity;
 
@@ -888,10 +891,14 @@ __global__ void clear_counters(uint32_t* counters, uint32_t* root_keys) {
 // References of the triangles and the root box, one atomic per workgroup and
 // coordinate on lines of their own (one per wave on one line took 380 us of
 // 352 k triangles' build).
+// A mesh's triangle with a vertex that is not finite has an infinite or NaN
+// determinant with every ray, which makes its inverse NaN and the triangle a
+// miss: its box is that of its finite coordinates, per axis, or 0.  Boxes of
+// instances (boxes set) stand for what is inside and stay as they are.
 __global__ void __launch_bounds__(256)
 make_refs(float const* __restrict__ positions, uint32_t stride, uint32_t num_vertices,
-          uint32_t const* __restrict__ indices, uint32_t num_triangles, Ref* __restrict__ refs,
-          uint32_t* __restrict__ root_keys, uint32_t* __restrict__ error) {
+          uint32_t const* __restrict__ indices, uint32_t num_triangles, uint32_t boxes,
+          Ref* __restrict__ refs, uint32_t* __restrict__ root_keys, uint32_t* __restrict__ error) {
     __shared__ float wave_lo[4][3];
     __shared__ float wave_hi[4][3];
 
@@ -917,12 +924,31 @@ make_refs(float const* __restrict__ positions, uint32_t stride, uint32_t num_ver
             // triangle_bvh_helper.cpp:15-21: min(a, min(b, c))
             r.lo[i] = smin(pa[i], smin(pb[i], pc[i]));
             r.hi[i] = smax(pa[i], smax(pb[i], pc[i]));
-            lo[i]   = fminf(lo[i], r.lo[i]);
-            hi[i]   = fmaxf(hi[i], r.hi[i]);
             finite  = finite && isfinite(pa[i]) && isfinite(pb[i]) && isfinite(pc[i]);
         }
-        if (!finite) {
+        if (!finite && boxes) {
             atomicOr(error, Not_finite);
+            for (int i = 0; i < 3; ++i) {  // one NaN, which sorts last (wave_sweep)
+                r.lo[i] = r.lo[i] != r.lo[i] ? __builtin_nanf("") : r.lo[i];
+                r.hi[i] = r.hi[i] != r.hi[i] ? __builtin_nanf("") : r.hi[i];
+            }
+        } else if (!finite) {
+            for (int i = 0; i < 3; ++i) {
+                float const v[3] = {pa[i], pb[i], pc[i]};
+                r.lo[i]          = Flt_max;
+                r.hi[i]          = -Flt_max;
+                for (int k = 0; k < 3; ++k) {
+                    r.lo[i] = isfinite(v[k]) ? smin(r.lo[i], v[k]) : r.lo[i];
+                    r.hi[i] = isfinite(v[k]) ? smax(r.hi[i], v[k]) : r.hi[i];
+                }
+                if (r.lo[i] > r.hi[i]) {
+                    r.lo[i] = r.hi[i] = 0.f;
+                }
+            }
+        }
+        for (int i = 0; i < 3; ++i) {
+            lo[i] = fminf(lo[i], r.lo[i]);
+            hi[i] = fmaxf(hi[i], r.hi[i]);
         }
         r.prim  = t;
         r.pad   = 0;
@@ -1081,7 +1107,7 @@ __device__ __forceinline__ Best wave_sweep(Task const& t, Ref const* refs, uint1
     }
 
     // each reference's place in the order of its max bound: (bound, index)
-    // ascending, -0 as +0, NaN last
+    // ascending, -0 as +0, NaN (without a sign, make_refs) last
     uint32_t own[3], rank[3] = {0, 0, 0}, less[3] = {0, 0, 0};
     for (int a = 0; a < 3; ++a) {
         own[a] = lane < n ? key(refs[lane].hi[a] + 0.f) : 0u;
@@ -1831,7 +1857,7 @@ struct Workspace {
 
 int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t position_stride,
                   uint32_t const* indices, uint32_t num_triangles, mi_bvh_settings const& settings,
-                  hipStream_t stream, DeviceBvh& out) {
+                  hipStream_t stream, DeviceBvh& out, bool boxes) {
     if (settings.sweep_threshold > 1024 || settings.num_slices > 64) {
         return fail(MI_ERR_ARGS, "mi_bvh_build: sweep_threshold <= 1024 and num_slices <= 64");
     }
@@ -1902,7 +1928,7 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
         MI_LAUNCHED();
         hipLaunchKernelGGL(make_refs, dim3(std::min(blocks_for(num_triangles, 256), 512u)), dim3(256),
                            0, st, positions, position_stride, num_vertices, indices, num_triangles,
-                           b.refs[0], root_keys, error);
+                           boxes ? 1u : 0u, b.refs[0], root_keys, error);
         MI_LAUNCHED();
         hipLaunchKernelGGL(init_root, dim3(1), dim3(256), 0, st, b, root_keys, num_triangles);
         MI_LAUNCHED();

@@ -11,9 +11,11 @@ namespace mi {
 // Builds the tree scene::shape::triangle::bvh::Builder_SAH builds
 // (triangle_bvh_builder_sah.cpp:21-67) from a device-resident mesh, on the
 // device, and lays it out depth-first as serialize() does.  Synchronous.
+// boxes: the triangles stand for instances' boxes (corners lo, hi, lo), which
+// are kept when they are not finite.
 int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t position_stride,
                   uint32_t const* indices, uint32_t num_triangles, mi_bvh_settings const& settings,
-                  hipStream_t stream, DeviceBvh& out);
+                  hipStream_t stream, DeviceBvh& out, bool boxes = false);
 
 // Frees the workspace kept between builds (mi_release).
 void release_build_workspace();

@@ -672,7 +672,8 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
         (void)hipFree(d_idx);
         return fail(MI_ERR_HIP, "instances: %s", hipGetErrorString(e));
     }
-    int32_t st = build_bvh(d_pos, 2 * num_instances, 3, d_idx, num_instances, settings, stream, out.tree);
+    int32_t st = build_bvh(d_pos, 2 * num_instances, 3, d_idx, num_instances, settings, stream, out.tree,
+                           true);
     (void)hipFree(d_pos);
     (void)hipFree(d_idx);
     if (st) {

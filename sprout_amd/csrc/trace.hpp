@@ -21,7 +21,7 @@ struct DeviceBvh {
     uint32_t num_slots     = 0;
     uint32_t num_triangles = 0;
     uint32_t max_depth     = 0;
-    bool     nan_bounds    = false;  // a vertex or node bound is not finite: no compressed pairs
+    bool     nan_bounds    = false;  // a node bound is not finite: no compressed pairs
 
     float  aabb_min[3] = {0.f, 0.f, 0.f};
     float  aabb_max[3] = {0.f, 0.f, 0.f};

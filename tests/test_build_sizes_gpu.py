@@ -59,6 +59,40 @@ def test_settings(gpu, settings, n):
     check(gpu, *soup(n, 7), **settings)
 
 
+def coordinates_not_finite(pos, value, triangles):
+    """value at a corner of each of the triangles of a soup, all three
+    corners on one axis for the last; and the soup whose boxes are those of
+    the finite coordinates"""
+    p = pos.reshape(-1, 3, 3).copy()
+    rng = np.random.default_rng(len(p))
+    at = rng.choice(len(p), triangles, replace=False)
+    for t in at[:-1]:
+        p[t, rng.integers(3), rng.integers(3)] = value
+    p[at[-1], :, 1] = value
+    q = p.copy()
+    for t in at:
+        for k in range(3):
+            ok = np.isfinite(p[t, :, k])
+            q[t, ~ok, k] = p[t, ok, k][0] if ok.any() else 0.0
+    return p.reshape(-1, 3), q.reshape(-1, 3)
+
+
+@pytest.mark.parametrize("value", [0x7FC00000, 0xFFC00000, 0x7F800000, 0xFF800000])
+@pytest.mark.parametrize("n", [1, 4, 20, 21, 64, 80, 1100, 5000])
+def test_vertices_not_finite(gpu, value, n):
+    """the tree of the finite coordinates, whatever the others' signs"""
+    import torch
+
+    print(f"{n} triangles, {value:08x}", flush=True)
+    pos, idx = soup(n, 3 * n)
+    p, q = coordinates_not_finite(pos, np.uint32(value).view(np.float32), min(n, 9))
+    tree = gpu.Builder_SAH().build(torch.from_numpy(p).cuda(), torch.from_numpy(idx.view(np.int32)).cuda())
+    nodes, slots = tree.download()
+    want = O.build(q, idx)
+    assert O.nodes_equal(nodes.view(O.NODE_DTYPE), want.nodes)
+    assert np.array_equal(slots, want.slots)
+
+
 def test_more_references_than_a_quarter_over(gpu):
     """a fifth of the triangles long: the levels outgrow the first two allocations"""
     pos, idx = soup(20000, 9, long=0.2)

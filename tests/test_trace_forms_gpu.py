@@ -126,7 +126,8 @@ def test_vertex_not_finite(gpu, mesh):
     agree(gpu, tree, rays_of(4096, 6))
 
 
-def test_hits_beside_a_vertex_not_finite(gpu, mesh):
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_hits_beside_a_vertex_not_finite(gpu, mesh, value):
     """the other triangles of such a mesh are hit as if it were not there,
     alone and instanced"""
     import torch
@@ -135,7 +136,7 @@ def test_hits_beside_a_vertex_not_finite(gpu, mesh):
 
     pos, idx, _ = mesh
     p = pos.copy()
-    p[7, 1] = p[300, 0] = np.nan
+    p[7, 1] = p[300, 0] = value
     tree = gpu.Builder_SAH().build(torch.from_numpy(p).cuda(),
                                    torch.from_numpy(idx.view(np.int32)).cuda())
     rays = rays_of(4096, 8)
