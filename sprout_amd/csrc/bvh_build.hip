@@ -469,6 +469,7 @@ struct Build {
 constexpr uint32_t Counter_nodes = Num_lc * Kind_words;  // word offsets
 constexpr uint32_t Counter_leafs = Counter_nodes + Line;
 constexpr uint32_t Counter_error = Counter_nodes + 2 * Line;
+constexpr uint32_t Counter_level = Counter_error + 1;  // of an unsplittable node
 constexpr uint32_t Build_words = Counter_nodes + 3 * Line;
 
 __device__ __forceinline__ uint32_t* counter(Build const& b, uint32_t level, uint32_t which) {
@@ -488,6 +489,12 @@ __device__ __forceinline__ bool stopped(Build const& b) {
     }
     __syncthreads();
     return 0 != (error & Err_stop);
+}
+
+// The levels after one with such a node are not built: one level writes here.
+__device__ __forceinline__ void unsplittable(Build const& b, uint32_t level) {
+    *counter(b, Counter_level) = level;
+    atomicOr(counter(b, Counter_error), Err_unsplittable);
 }
 
 __device__ __forceinline__ uint32_t bin_words(Build const& b) {
@@ -1235,7 +1242,7 @@ wave_nodes(Build b, uint32_t level) {
                 if (0 == lane) {
                     decision_s[i] = d;
                     if (Kind_error == d.kind) {
-                        atomicOr(counter(b, Counter_error), Err_unsplittable);
+                        unsplittable(b, level);
                     }
                 }
             }
@@ -1333,7 +1340,7 @@ __device__ __forceinline__ bool take_places(Build const& b, uint32_t level, Task
             s.full = 1;
         }
         if (0 == threadIdx.x && Kind_error == d.kind) {
-            atomicOr(counter(b, Counter_error), Err_unsplittable);
+            unsplittable(b, level);
         }
     }
     __syncthreads();
@@ -1992,7 +1999,7 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
             return fail(MI_ERR_UNSPLITTABLE,
                         "mi_bvh_build: a node of more than 255 references cannot be split "
                         "(level %u)",
-                        level ? level - 1 : 0);
+                        host[Counter_level]);
         }
         if (err & Err_capacity) {
             continue;

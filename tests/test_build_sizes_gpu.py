@@ -59,6 +59,22 @@ def test_settings(gpu, settings, n):
     check(gpu, *soup(n, 7), **settings)
 
 
+@pytest.mark.parametrize("level", [0, 1])
+def test_the_level_of_an_unsplittable_node(gpu, level):
+    """300 times one triangle, alone or beside a soup that the root splits off"""
+    import torch
+
+    from sprout_amd import _lib
+
+    one = np.array([[0, 0, 0], [0.1, 0, 0], [0, 0.1, 0.1]], np.float32)
+    pos = np.tile(one, (300, 1))
+    if level:
+        pos = np.concatenate([pos, soup(600, 5)[0] + np.float32(50)])
+    idx = np.arange(len(pos), dtype=np.int32).reshape(-1, 3)
+    with pytest.raises(_lib.MiError, match=rf"cannot be split \(level {level}\)"):
+        gpu.Builder_SAH().build(torch.from_numpy(pos).cuda(), torch.from_numpy(idx).cuda())
+
+
 def coordinates_not_finite(pos, value, triangles):
     """value at a corner of each of the triangles of a soup, all three
     corners on one axis for the last; and the soup whose boxes are those of
