@@ -1072,7 +1072,7 @@ int32_t launch(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays, ui
         spill   = fixed->spill;
         counter = fixed->counter;
     } else {
-        if (int32_t const st = res.reserve_spill(lane_words * blocks * block); st) {
+        if (int32_t const st = res.reserve_spill(lane_words * res.max_blocks(num_rays) * block); st) {
             return st;
         }
         spill   = res.spill;
@@ -1204,7 +1204,7 @@ int32_t prepare_trace(DeviceBvh const& bvh, TraceResources& res, uint32_t max_ra
                     "tree depth %u needs %u stack entries, more than the reference's %u",
                     bvh.max_depth, entries, Reference_stack_size);
     }
-    uint32_t const     threads = res.grid_blocks(max_rays) * res.block_size;
+    uint32_t const     threads = res.max_blocks(max_rays) * res.block_size;
     Stack_layout const sl      = stack_layout(bvh, res, false);
     if (4 == res.kernel && 2 == sl.words) {
         // made before any capture: a launch inside a graph allocates nothing

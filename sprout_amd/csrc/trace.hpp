@@ -84,6 +84,17 @@ struct TraceResources {
         return uint32_t(b > 0 ? b : 1);
     }
 
+    // The most workgroups of any launch of up to max_rays rays.  Its own grid
+    // may be smaller: up to spread_waves() rays take a wave each, a few more
+    // take two or three a wave.  Stack areas are sized by this, so a launch
+    // never needs more than a larger one before it (which may be captured, or
+    // reserve for a capture).
+    uint32_t max_blocks(uint32_t max_rays) const {
+        uint32_t const spread = grid_blocks(max_rays < spread_waves() ? max_rays : spread_waves());
+        uint32_t const own    = grid_blocks(max_rays);
+        return spread > own ? spread : own;
+    }
+
     int32_t reserve_spill(size_t words);
 
     void release();

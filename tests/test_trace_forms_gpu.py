@@ -239,3 +239,31 @@ def test_origins_on_bounds_of_instances(gpu):
         assert np.array_equal(got if any_hit else got[:, :5], want), any_hit
     assert want.mean() > 0.05
     inst.release()
+
+
+def test_captured_launch_after_a_smaller_one(gpu, mesh):
+    """a captured launch's stack area stays its own when a smaller launch,
+    with more waves, follows: replays give the same hits"""
+    import torch
+
+    pos, idx, otree = mesh
+    tree = gpu.upload(otree.nodes, otree.slots, pos, idx)
+    gpu.set_trace_config(lds_entries=1)  # every walk spills
+    d = torch.from_numpy(rays_of(5000, 31)).cuda()
+    small = d[:4000].contiguous()
+    want = tree.intersect(d).clone()  # reserves
+    hits = torch.empty_like(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tree.intersect(d, hits)
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        tree.intersect(small)  # nothing is allocated inside a capture
+    for _ in range(3):
+        assert torch.equal(tree.intersect(small), want[:4000])
+        hits.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(hits, want)
+    gpu.set_trace_config()
+    assert torch.equal(tree.counts(d)[0], want)
