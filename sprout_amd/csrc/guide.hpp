@@ -12,6 +12,7 @@
 #pragma once
 
 #include "bsdf.hpp"
+#include "launch_key.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -68,6 +69,12 @@ struct GuideNet {
 
     void release();
 };
+
+// What captured launches of a network hold of it.
+inline void put_guide_key(Launch_key& key, GuideNet const& n) {
+    put_key(key, n.params, n.adam_m, n.adam_v, n.grad, n.partial, n.wsum, n.freq, n.wt, n.window,
+            n.step_dev, n.scratch_step, n.partial_blocks);
+}
 
 int32_t guide_create(uint64_t seed, uint32_t num_cus, GuideNet& out);
 int32_t guide_set_params(GuideNet& net, float const* host_params);

@@ -93,6 +93,13 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
                     uint32_t num_instances, mi_bvh_settings const& settings, hipStream_t stream,
                     Tlas& out);
 
+// What a captured trace_instances_launch holds besides its arguments: the view
+// and the stack area, whose size sets the grid (none: the one-word kernel).
+inline void put_instances_key(Launch_key& key, Tlas const& t) {
+    put_key(key, t.tree.nodes, t.tree.tris, t.tree.num_nodes, t.instances, t.meshes, t.spill,
+            t.spill_total, t.claims);
+}
+
 // Closest (out: mi_instance_hit per ray, pad[0] = the mesh tree's slot) or
 // any hit (out: uint32 per ray).  n_dev (optional): a ray count in device
 // memory, at most n (capturable).  claims (optional): ray claim counters

@@ -3950,6 +3950,16 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
         return MI_OK;
     };
 
+    // what the kernels of a bounce hold when they are captured
+    auto bounce_key = [&]() -> Launch_key {
+        Launch_key key(sizeof(Wave));
+        std::memcpy(key.data(), &w, sizeof(Wave));
+        put_key(key, grid_path, num_shadow);
+        put_trace_key(key, scene.bvh, trace);
+        put_instances_key(key, scene.tlas);
+        return key;
+    };
+
     // order after the caller's earlier work on its stream
     hipError_t e = hipEventRecord(state.begin, stream);
     if (!e) e = hipStreamWaitEvent(s, state.begin, 0);
@@ -3977,24 +3987,7 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
             (uint64_t(set.max_bounces) + 2) * ((batch_samples + live_slots - 1) / live_slots + 1) + 8;
         bool const use_graph = 0 == (set.flags & MI_RENDER_NO_GRAPH);
         if (use_graph) {
-            std::vector<uint8_t> key(sizeof(Wave));
-            std::memcpy(key.data(), &w, sizeof(Wave));
-            auto put = [&key](auto const& v) {
-                uint8_t const* b = reinterpret_cast<uint8_t const*>(&v);
-                key.insert(key.end(), b, b + sizeof(v));
-            };
-            put(grid_path);
-            put(num_shadow);
-            put(scene.bvh.nodes);
-            put(scene.bvh.tris);
-            put(trace.counter);
-            put(trace.spill);
-            put(trace.lds_entries);
-            put(trace.kernel);
-            put(trace.block_size);
-            put(trace.blocks_per_cu);
-            put(trace.refill_lanes);
-            put(trace.claim_batch);
+            Launch_key key = bounce_key();
             if (!state.regen_graph || key != state.regen_key) {
                 if (state.regen_graph) {
                     (void)hipStreamSynchronize(s);
@@ -4084,35 +4077,14 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
         // comes a second time running, or for many waves: with the camera
         // moved each frame, frames of 1 / 4 / 16 waves of 97x61 took 0.60 /
         // 1.95 / 7.38 ms captured and 0.49 / 1.88 / 7.43 ms launched.
-        std::vector<uint8_t> key(sizeof(Wave));
-        std::memcpy(key.data(), &w, sizeof(Wave));
-        auto put = [&key](auto const& v) {
-            uint8_t const* b = reinterpret_cast<uint8_t const*>(&v);
-            key.insert(key.end(), b, b + sizeof(v));
-        };
-        put(accum);
-        put(sensor != nullptr);  // which resolve ends the wave
-        put(grid_path);
-        put(num_shadow);
-        put(spw);
-        put(scene.bvh.nodes);
-        put(scene.bvh.tris);
-        put(trace.counter);
-        put(trace.spill);
-        put(trace.lds_entries);
-        put(trace.kernel);
-        put(trace.block_size);
-        put(trace.blocks_per_cu);
-        put(trace.refill_lanes);
-        put(trace.claim_batch);
-        put(training);
-        put(net);
+        Launch_key key = bounce_key();
+        put_key(key, accum, sensor != nullptr /* which resolve ends the wave */, spw, training, net);
+        if (guided) {
+            put_guide_key(key, *net);
+        }
         if (training) {
-            put(gs->train_steps);
-            put(gs->batch);
-            put(gs->learning_rate);
-            put(records);
-            put(state.shuf_x);
+            put_key(key, gs->train_steps, gs->batch, gs->learning_rate, records, state.shuf_x,
+                    state.shuf_dir, state.shuf_w);
         }
         bool const cached  = state.graph && key == state.graph_key;
         bool const capture = !cached && (key == state.last_key || waves >= Capture_waves);

@@ -211,8 +211,8 @@ struct RenderState {
     hipEvent_t   begin       = nullptr;
     hipEvent_t   end         = nullptr;
     hipGraphExec_t       graph = nullptr;  // the last wave's graph, replayed while its key holds
-    std::vector<uint8_t> graph_key;
-    std::vector<uint8_t> last_key;         // the last wave's, captured or not
+    Launch_key           graph_key;
+    Launch_key           last_key;         // the last wave's, captured or not
     // guiding
     uint32_t  guide_capacity  = 0;
     float*    guide_x         = nullptr;  // network inputs per queue entry
@@ -234,7 +234,7 @@ struct RenderState {
     uint32_t  done_capacity   = 0;
     uint32_t* live_host       = nullptr;  // pinned: the next queue's length after a graph replay
     hipGraphExec_t       regen_graph = nullptr;  // two regenerating bounces, replayed while its key holds
-    std::vector<uint8_t> regen_key;
+    Launch_key           regen_key;
     float2*   path_spec       = nullptr;  // spectral: per path slot {fourth throughput, hero}
     float*    nee_thr4        = nullptr;  // spectral: per queue entry
     uint32_t  spectral_capacity = 0;

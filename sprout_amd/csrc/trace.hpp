@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "launch_key.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -127,6 +128,17 @@ int32_t prepare_trace(DeviceBvh const& bvh, TraceResources& res, uint32_t max_ra
 int32_t launch_trace_device_count(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays,
                                   uint32_t const* num_rays, uint32_t max_rays, void* out,
                                   bool any_hit, hipStream_t stream, uint32_t* claims);
+
+// What a captured launch_trace_device_count holds besides its arguments: the
+// tree (its addresses come back with other trees, whose depth sets the stack's
+// split between LDS and the spill area and whose size or pairs set the
+// kernel), the launch shape and the context's buffers.
+inline void put_trace_key(Launch_key& key, DeviceBvh const& bvh, TraceResources const& res) {
+    put_key(key, bvh.nodes, bvh.tris, bvh.num_nodes, bvh.num_slots, bvh.max_depth, bvh.nan_bounds,
+            bvh.qpairs, bvh.qorigin, bvh.qscale);
+    put_key(key, res.counter, res.spill, res.lds_entries, res.kernel, res.block_size,
+            res.blocks_per_cu, res.num_cus, res.refill_lanes, res.claim_batch);
+}
 
 // Sets up the fixed scratch of launch_trace_noalloc on `device`, which must
 // be the current device (once per device; later calls return at once).
