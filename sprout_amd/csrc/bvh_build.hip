@@ -51,6 +51,7 @@
 
 #include "bvh_build.hpp"
 #include "device_math.hpp"
+#include "device_memory.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -1768,8 +1769,9 @@ uint32_t blocks_for(uint64_t n, uint32_t block) {
 
 // A build's workspace (one device allocation) and the page-locked words its
 // counters are read into.  The last build's are kept for the next one on
-// the same device, up to Keep_bytes, until mi_release: allocating and freeing
-// took about as long as a small build.  A build that finds them in use by
+// the same device, up to Keep_bytes, until mi_release or until the device's
+// memory is used up (device_malloc): allocating and freeing took about as long
+// as a small build.  A build that finds them in use by
 // another thread has its own; one that ends early gives its own back, since
 // its kernels may still run.
 constexpr size_t Keep_bytes = size_t(1) << 30;
@@ -1829,7 +1831,7 @@ struct Workspace {
             (void)hipFree(base);
             base  = nullptr;
             bytes = 0;
-            e     = hipMalloc(&base, n);
+            e     = device_malloc(&base, n);
             if (!e) {
                 bytes = n;
             }
@@ -2023,12 +2025,12 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
         bvh.num_triangles = num_triangles;
         bvh.max_depth     = deepest;
 
-        hipError_t e = hipMalloc(&bvh.nodes_alloc, size_t(bvh.num_nodes + 1) * 32);
+        hipError_t e = device_malloc(&bvh.nodes_alloc, size_t(bvh.num_nodes + 1) * 32);
         if (e == hipSuccess) {
-            e = hipMalloc(&bvh.tris, size_t(std::max(1u, bvh.num_slots)) * 48);
+            e = device_malloc(&bvh.tris, size_t(std::max(1u, bvh.num_slots)) * 48);
         }
         if (e == hipSuccess) {
-            e = hipMalloc(&bvh.slots, size_t(std::max(1u, bvh.num_slots)) * 4);
+            e = device_malloc(&bvh.slots, size_t(std::max(1u, bvh.num_slots)) * 4);
         }
         if (e != hipSuccess) {
             bvh.release();
@@ -2082,8 +2084,9 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
     }
 }
 
-void release_build_workspace() {
+bool release_build_workspace() {
     std::lock_guard<std::mutex> guard(kept.lock);
+    bool const any = nullptr != kept.base;
     (void)hipFree(kept.base);
     if (kept.words) {
         (void)hipHostFree(kept.words);
@@ -2092,6 +2095,7 @@ void release_build_workspace() {
     kept.base   = nullptr;
     kept.bytes  = 0;
     kept.words  = nullptr;
+    return any;
 }
 
 }  // namespace mi

@@ -17,7 +17,4 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
                   uint32_t const* indices, uint32_t num_triangles, mi_bvh_settings const& settings,
                   hipStream_t stream, DeviceBvh& out, bool boxes = false);
 
-// Frees the workspace kept between builds (mi_release).
-void release_build_workspace();
-
 }  // namespace mi

@@ -2,6 +2,7 @@
 // per-slot triangle records the traversal reads.
 
 #include "common.hpp"
+#include "device_memory.hpp"
 #include "trace.hpp"
 
 #include <hip/hip_runtime.h>
@@ -66,7 +67,7 @@ int32_t TraceResources::reserve_spill(size_t words) {
     (void)hipFree(spill);
     spill       = nullptr;
     spill_words = 0;
-    if (hipError_t const e = hipMalloc(&spill, words * sizeof(uint32_t)); e != hipSuccess) {
+    if (hipError_t const e = device_malloc(&spill, words * sizeof(uint32_t)); e != hipSuccess) {
         return fail(MI_ERR_HIP, "spill stack allocation of %zu words: %s", words,
                     hipGetErrorString(e));
     }
@@ -162,18 +163,18 @@ int32_t upload_bvh(void const* nodes, uint32_t num_nodes, uint32_t const* slots,
     size_t const pos_bytes = size_t(num_vertices) * position_stride * sizeof(float);
     size_t const idx_bytes = size_t(num_triangles) * 3 * sizeof(uint32_t);
 
-    hipError_t e = hipMalloc(&bvh.nodes_alloc, size_t(num_nodes + 1) * 32);
+    hipError_t e = device_malloc(&bvh.nodes_alloc, size_t(num_nodes + 1) * 32);
     if (e == hipSuccess) {
-        e = hipMalloc(&bvh.tris, size_t(num_slots ? num_slots : 1) * 48);
+        e = device_malloc(&bvh.tris, size_t(num_slots ? num_slots : 1) * 48);
     }
     if (e == hipSuccess) {
-        e = hipMalloc(&bvh.slots, size_t(num_slots ? num_slots : 1) * 4);
+        e = device_malloc(&bvh.slots, size_t(num_slots ? num_slots : 1) * 4);
     }
     if (e == hipSuccess) {
-        e = hipMalloc(&d_pos, pos_bytes ? pos_bytes : 4);
+        e = device_malloc(&d_pos, pos_bytes ? pos_bytes : 4);
     }
     if (e == hipSuccess) {
-        e = hipMalloc(&d_idx, idx_bytes ? idx_bytes : 4);
+        e = device_malloc(&d_idx, idx_bytes ? idx_bytes : 4);
     }
     if (e == hipSuccess) {
         bvh.nodes = reinterpret_cast<float4*>(static_cast<char*>(bvh.nodes_alloc) + 32);

@@ -2,6 +2,7 @@
 
 #include "bvh_build.hpp"
 #include "common.hpp"
+#include "device_memory.hpp"
 #include "guide.hpp"
 #include "instances.hpp"
 #include "light_build.hip.hpp"
@@ -145,7 +146,7 @@ int32_t mi_init(int32_t device) {
     }
 
     uint32_t* counter = nullptr;
-    if (hipError_t const e = hipMalloc(&counter, Counter_words * sizeof(uint32_t)); e != hipSuccess) {
+    if (hipError_t const e = device_malloc(&counter, Counter_words * sizeof(uint32_t)); e != hipSuccess) {
         return fail(MI_ERR_HIP, "mi_init: %s", hipGetErrorString(e));
     }
 
@@ -414,7 +415,7 @@ int32_t mi_trace_autotune(uint32_t bvh, mi_ray const* rays, uint32_t num_rays, u
     hipStream_t const s    = as_stream(stream);
     mi_hit*           hits = nullptr;
     hipEvent_t        e0 = nullptr, e1 = nullptr;
-    hipError_t        e  = hipMalloc(&hits, size_t(num_rays) * sizeof(mi_hit));
+    hipError_t        e  = device_malloc(&hits, size_t(num_rays) * sizeof(mi_hit));
     if (!e) e = hipEventCreate(&e0);
     if (!e) e = hipEventCreate(&e1);
     if (e) {
@@ -486,7 +487,7 @@ int32_t mi_trace_autotune(uint32_t bvh, mi_ray const* rays, uint32_t num_rays, u
         hipError_t fe = hipEventCreate(&f0);
         if (!fe) fe = hipEventCreate(&f1);
         mi_hit* sh = nullptr;
-        if (!fe) fe = hipMalloc(&sh, size_t(num_rays) * sizeof(mi_hit));
+        if (!fe) fe = device_malloc(&sh, size_t(num_rays) * sizeof(mi_hit));
         t.sort_rays = 1;
         int32_t fs  = fe ? MI_ERR_HIP : launch_trace(*b, t, rays, num_rays, sh, nullptr, false, s);
         if (!fs && !fe) fe = hipEventRecord(f0, s);
@@ -680,7 +681,7 @@ int32_t render_call(uint32_t scene, mi_camera const* camera, mi_render_settings 
     }
     TraceResources& rt = context->render_trace;
     if (!rt.counter) {
-        if (hipError_t const e = hipMalloc(&rt.counter, Counter_words * sizeof(uint32_t)); e) {
+        if (hipError_t const e = device_malloc(&rt.counter, Counter_words * sizeof(uint32_t)); e) {
             return fail(MI_ERR_HIP, "mi_render: %s", hipGetErrorString(e));
         }
     }

@@ -23,6 +23,7 @@
 // adam      one thread per parameter; refreshes the bf16 W^T copy.
 
 #include "common.hpp"
+#include "device_memory.hpp"
 #include "guide.hpp"
 
 #include <hip/hip_runtime.h>
@@ -882,20 +883,20 @@ void GuideNet::release() {
 int32_t guide_create(uint64_t seed, uint32_t num_cus, GuideNet& out) {
     GuideNet n;
     n.partial_blocks = num_cus ? num_cus : 256;
-    hipError_t e     = hipMalloc(&n.params, Num_params * sizeof(float));
-    if (!e) e = hipMalloc(&n.adam_m, Num_params * sizeof(float));
-    if (!e) e = hipMalloc(&n.adam_v, Num_params * sizeof(float));
-    if (!e) e = hipMalloc(&n.grad, Num_params * sizeof(float));
-    if (!e) e = hipMalloc(&n.partial, size_t(n.partial_blocks) * Num_params * sizeof(float));
-    if (!e) e = hipMalloc(&n.wsum, size_t(n.partial_blocks) * sizeof(float));
-    if (!e) e = hipMalloc(&n.freq, Num_in * Num_freq * sizeof(float));
+    hipError_t e     = device_malloc(&n.params, Num_params * sizeof(float));
+    if (!e) e = device_malloc(&n.adam_m, Num_params * sizeof(float));
+    if (!e) e = device_malloc(&n.adam_v, Num_params * sizeof(float));
+    if (!e) e = device_malloc(&n.grad, Num_params * sizeof(float));
+    if (!e) e = device_malloc(&n.partial, size_t(n.partial_blocks) * Num_params * sizeof(float));
+    if (!e) e = device_malloc(&n.wsum, size_t(n.partial_blocks) * sizeof(float));
+    if (!e) e = device_malloc(&n.freq, Num_in * Num_freq * sizeof(float));
     if (!e) {
         float f[Num_in * Num_freq];
         guide_default_frequencies(f);
         e = hipMemcpy(n.freq, f, sizeof(f), hipMemcpyHostToDevice);
     }
-    if (!e) e = hipMalloc(&n.wt, Num_t * sizeof(uint16_t));
-    if (!e) e = hipMalloc(&n.window, 8 * sizeof(uint32_t));
+    if (!e) e = device_malloc(&n.wt, Num_t * sizeof(uint16_t));
+    if (!e) e = device_malloc(&n.window, 8 * sizeof(uint32_t));
     if (e) {
         n.release();
         return fail(MI_ERR_HIP, "guide: %s", hipGetErrorString(e));

@@ -24,6 +24,7 @@
 
 #include "claims.hpp"
 #include "device_math.hpp"
+#include "device_memory.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -663,8 +664,8 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
 
     float*    d_pos = nullptr;
     uint32_t* d_idx = nullptr;
-    hipError_t e    = hipMalloc(&d_pos, pos.size() * sizeof(float));
-    if (!e) e = hipMalloc(&d_idx, idx.size() * sizeof(uint32_t));
+    hipError_t e    = device_malloc(&d_pos, pos.size() * sizeof(float));
+    if (!e) e = device_malloc(&d_idx, idx.size() * sizeof(uint32_t));
     if (!e) e = hipMemcpy(d_pos, pos.data(), pos.size() * sizeof(float), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(d_idx, idx.data(), idx.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (e) {
@@ -695,8 +696,8 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
         views[k].nodes = meshes[k]->nodes;
         views[k].tris  = meshes[k]->tris;
     }
-    e = hipMalloc(&out.instances, num_instances * sizeof(Instance_record));
-    if (!e) e = hipMalloc(&out.meshes, num_meshes * sizeof(Mesh_view));
+    e = device_malloc(&out.instances, num_instances * sizeof(Instance_record));
+    if (!e) e = device_malloc(&out.meshes, num_meshes * sizeof(Mesh_view));
     if (!e) e = hipMemcpy(out.instances, out.records.data(), num_instances * sizeof(Instance_record),
                           hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(out.meshes, views.data(), num_meshes * sizeof(Mesh_view), hipMemcpyHostToDevice);
@@ -720,8 +721,8 @@ int32_t create_tlas(DeviceBvh const* const* meshes, uint32_t num_meshes, uint32_
         if (!e) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
         uint32_t const total  = uint32_t(std::max(cus, 1)) * Blocks_per_cu * Block2;
         uint32_t const deeper = out.max_stack > Lds_entries ? out.max_stack - Lds_entries : 0;
-        if (!e) e = hipMalloc(&out.spill, std::max<size_t>(1, size_t(2) * deeper * total) * sizeof(uint32_t));
-        if (!e) e = hipMalloc(&out.claims, Counter_words * sizeof(uint32_t));
+        if (!e) e = device_malloc(&out.spill, std::max<size_t>(1, size_t(2) * deeper * total) * sizeof(uint32_t));
+        if (!e) e = device_malloc(&out.claims, Counter_words * sizeof(uint32_t));
         if (e) {
             out.release();
             return fail(MI_ERR_HIP, "instances: stack area: %s", hipGetErrorString(e));

@@ -32,6 +32,7 @@
 #include "light_build.hip.hpp"
 
 #include "light_build.hpp"
+#include "device_memory.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -751,15 +752,15 @@ int32_t Light_forest_scratch::reserve(uint32_t lights, uint32_t roots) {
     uint32_t const nr = std::max(roots, root_capacity);
     release();
     size_t const counter_words = 4 + Max_levels + 2;
-    hipError_t   e = hipMalloc(&recs, size_t(nl) * sizeof(Rec));
-    if (!e) e = hipMalloc(&owner, size_t(nl) * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&sides, 3 * size_t(nl) * sizeof(lb::Sides));
-    if (!e) e = hipMalloc(&nodes, (2 * size_t(nl) + 1) * sizeof(Tnode));
-    if (!e) e = hipMalloc(&counters, counter_words * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&swap_left, size_t(nl) * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&swap_right, size_t(nl) * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&num_nodes, size_t(nr + 1) * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&first, size_t(nr + 1) * sizeof(uint32_t));
+    hipError_t   e = device_malloc(&recs, size_t(nl) * sizeof(Rec));
+    if (!e) e = device_malloc(&owner, size_t(nl) * sizeof(uint32_t));
+    if (!e) e = device_malloc(&sides, 3 * size_t(nl) * sizeof(lb::Sides));
+    if (!e) e = device_malloc(&nodes, (2 * size_t(nl) + 1) * sizeof(Tnode));
+    if (!e) e = device_malloc(&counters, counter_words * sizeof(uint32_t));
+    if (!e) e = device_malloc(&swap_left, size_t(nl) * sizeof(uint32_t));
+    if (!e) e = device_malloc(&swap_right, size_t(nl) * sizeof(uint32_t));
+    if (!e) e = device_malloc(&num_nodes, size_t(nr + 1) * sizeof(uint32_t));
+    if (!e) e = device_malloc(&first, size_t(nr + 1) * sizeof(uint32_t));
     // page-locked: the counters, then the roots' offsets and node counts
     if (!e) e = hipHostMalloc(&host, (counter_words + size_t(nr + 1)) * sizeof(uint32_t));
     if (e) {

@@ -41,6 +41,7 @@
 #include "bvh_build.hpp"
 #include "common.hpp"
 #include "device_math.hpp"
+#include "device_memory.hpp"
 #include "guide.hpp"
 #include "light_build.hip.hpp"
 #include "light_build.hpp"
@@ -2161,7 +2162,7 @@ bool is_light(mi_material const& m) {
 
 int32_t make_energy_table(float** table) {
     float* t = nullptr;
-    if (hipError_t const e = hipMalloc(&t, dev::E_size * dev::E_size * sizeof(float)); e) {
+    if (hipError_t const e = device_malloc(&t, dev::E_size * dev::E_size * sizeof(float)); e) {
         return fail(MI_ERR_HIP, "energy table: %s", hipGetErrorString(e));
     }
     hipLaunchKernelGGL(energy_table, dim3(dev::E_size * dev::E_size), dim3(256), 0, nullptr, t);
@@ -2336,7 +2337,7 @@ int32_t upload_unit_normals(float const* normals, uint32_t num_vertices, float**
     float*     p = *d;
     hipError_t e = hipSuccess;
     if (!p) {
-        e = hipMalloc(&p, unit.size() * sizeof(float));
+        e = device_malloc(&p, unit.size() * sizeof(float));
     }
     if (!e) e = hipMemcpy(p, unit.data(), unit.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e) {
@@ -2470,9 +2471,9 @@ int32_t set_medium(RenderScene& scene, float const* density, uint32_t const dims
         }
     }
 
-    hipError_t e = hipMalloc(&scene.medium_density, n * sizeof(float));
-    if (!e) e = hipMalloc(&scene.medium_levels, levels.size());
-    if (!e) e = hipMalloc(&scene.medium_leaves, leaves.size() * sizeof(Medium_cm));
+    hipError_t e = device_malloc(&scene.medium_density, n * sizeof(float));
+    if (!e) e = device_malloc(&scene.medium_levels, levels.size());
+    if (!e) e = device_malloc(&scene.medium_leaves, leaves.size() * sizeof(Medium_cm));
     if (!e) e = hipMemcpy(scene.medium_density, density, n * sizeof(float), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(scene.medium_levels, levels.data(), levels.size(), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(scene.medium_leaves, leaves.data(), leaves.size() * sizeof(Medium_cm),
@@ -2697,16 +2698,16 @@ int32_t create_scene(float const* positions, uint32_t num_vertices, uint32_t con
 
     size_t const nl = std::max<size_t>(1, infos.size());
     size_t const nn = std::max<size_t>(1, 2 * infos.size());  // room for any tree over the parts
-    hipError_t   e  = hipMalloc(&s.positions, size_t(num_vertices) * 3 * sizeof(float));
-    if (!e) e = hipMalloc(&s.indices, size_t(num_triangles) * 3 * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&s.tri_material, size_t(num_triangles) * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&s.materials, std::max<size_t>(1, num_materials) * sizeof(Render_material));
-    if (!e) e = hipMalloc(&s.light_nodes, nn * sizeof(Light_node));
-    if (!e) e = hipMalloc(&s.light_middles, nn * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&s.light_mapping, nl * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&s.light_orders, nl * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&s.light_infos, nl * sizeof(Light_info));
-    if (!e) e = hipMalloc(&s.tri_light, size_t(num_triangles) * sizeof(uint32_t));
+    hipError_t   e  = device_malloc(&s.positions, size_t(num_vertices) * 3 * sizeof(float));
+    if (!e) e = device_malloc(&s.indices, size_t(num_triangles) * 3 * sizeof(uint32_t));
+    if (!e) e = device_malloc(&s.tri_material, size_t(num_triangles) * sizeof(uint32_t));
+    if (!e) e = device_malloc(&s.materials, std::max<size_t>(1, num_materials) * sizeof(Render_material));
+    if (!e) e = device_malloc(&s.light_nodes, nn * sizeof(Light_node));
+    if (!e) e = device_malloc(&s.light_middles, nn * sizeof(uint32_t));
+    if (!e) e = device_malloc(&s.light_mapping, nl * sizeof(uint32_t));
+    if (!e) e = device_malloc(&s.light_orders, nl * sizeof(uint32_t));
+    if (!e) e = device_malloc(&s.light_infos, nl * sizeof(Light_info));
+    if (!e) e = device_malloc(&s.tri_light, size_t(num_triangles) * sizeof(uint32_t));
     if (!e) e = hipMemcpy(s.positions, positions, size_t(num_vertices) * 3 * sizeof(float), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(s.indices, indices, size_t(num_triangles) * 3 * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(s.tri_material, tri_material, size_t(num_triangles) * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -2723,7 +2724,7 @@ int32_t create_scene(float const* positions, uint32_t num_vertices, uint32_t con
     auto upload = [&e](auto*& dst, auto const& v) {
         using T = std::remove_reference_t<decltype(v[0])>;
         size_t const bytes = std::max<size_t>(1, v.size()) * sizeof(T);
-        if (!e) e = hipMalloc(reinterpret_cast<void**>(&dst), bytes);
+        if (!e) e = device_malloc(reinterpret_cast<void**>(&dst), bytes);
         if (!e && !v.empty()) e = hipMemcpy(dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice);
     };
     upload(s.part_infos, pinfo);
@@ -2962,19 +2963,19 @@ int32_t update_positions(RenderScene& s, float const* positions, uint32_t num_ve
     if (N > w.capacity_tris || P > w.capacity_parts || !w.bad) {
         w.release();
         size_t const n = std::max<size_t>(1, N), p = std::max<size_t>(1, P);
-        e = hipMalloc(&w.tri_lo, 3 * n * sizeof(float));
-        if (!e) e = hipMalloc(&w.tri_hi, 3 * n * sizeof(float));
-        if (!e) e = hipMalloc(&w.tri_cone, 4 * n * sizeof(float));
-        if (!e) e = hipMalloc(&w.tri_power, n * sizeof(float));
-        if (!e) e = hipMalloc(&w.part_cone, 4 * p * sizeof(float));
-        if (!e) e = hipMalloc(&w.part_lo, 3 * p * sizeof(float));
-        if (!e) e = hipMalloc(&w.part_hi, 3 * p * sizeof(float));
-        if (!e) e = hipMalloc(&w.part_pow, p * sizeof(float));
-        if (!e) e = hipMalloc(&w.part_two, p);
-        if (!e) e = hipMalloc(&w.cdf_rel, 2 * n * sizeof(uint32_t));
-        if (!e) e = hipMalloc(&w.num_cdfs, p * sizeof(uint32_t));
-        if (!e) e = hipMalloc(&w.part_first, (p + 1) * sizeof(uint32_t));
-        if (!e) e = hipMalloc(&w.bad, sizeof(uint32_t));
+        e = device_malloc(&w.tri_lo, 3 * n * sizeof(float));
+        if (!e) e = device_malloc(&w.tri_hi, 3 * n * sizeof(float));
+        if (!e) e = device_malloc(&w.tri_cone, 4 * n * sizeof(float));
+        if (!e) e = device_malloc(&w.tri_power, n * sizeof(float));
+        if (!e) e = device_malloc(&w.part_cone, 4 * p * sizeof(float));
+        if (!e) e = device_malloc(&w.part_lo, 3 * p * sizeof(float));
+        if (!e) e = device_malloc(&w.part_hi, 3 * p * sizeof(float));
+        if (!e) e = device_malloc(&w.part_pow, p * sizeof(float));
+        if (!e) e = device_malloc(&w.part_two, p);
+        if (!e) e = device_malloc(&w.cdf_rel, 2 * n * sizeof(uint32_t));
+        if (!e) e = device_malloc(&w.num_cdfs, p * sizeof(uint32_t));
+        if (!e) e = device_malloc(&w.part_first, (p + 1) * sizeof(uint32_t));
+        if (!e) e = device_malloc(&w.bad, sizeof(uint32_t));
         if (!e && P) {
             e = hipMemcpy(w.part_first, s.part_first.data(), (P + 1) * sizeof(uint32_t),
                           hipMemcpyHostToDevice);
@@ -2989,7 +2990,7 @@ int32_t update_positions(RenderScene& s, float const* positions, uint32_t num_ve
     // the new positions, checked before the scene takes them: every
     // emissive triangle must keep an area
     float* fresh = nullptr;
-    e            = hipMalloc(&fresh, std::max<size_t>(1, num_vertices) * 3 * sizeof(float));
+    e            = device_malloc(&fresh, std::max<size_t>(1, num_vertices) * 3 * sizeof(float));
     if (!e) e = hipMemcpyAsync(fresh, positions, size_t(num_vertices) * 3 * sizeof(float),
                                hipMemcpyDeviceToDevice, stream);
     if (!e) e = hipMemsetAsync(w.bad, 0, sizeof(uint32_t), stream);
@@ -3170,9 +3171,9 @@ int32_t create_scene_instanced(mi_mesh const* meshes, uint32_t num_meshes,
         mi_mesh const& m   = meshes[k];
         float*         pos = nullptr;
         uint32_t*      idx = nullptr;
-        hipError_t     e   = hipMalloc(&pos, size_t(m.num_vertices) * 3 * sizeof(float));
+        hipError_t     e   = device_malloc(&pos, size_t(m.num_vertices) * 3 * sizeof(float));
         if (!e) s.mesh_buffers.push_back(pos);
-        if (!e) e = hipMalloc(&idx, size_t(m.num_triangles) * 3 * sizeof(uint32_t));
+        if (!e) e = device_malloc(&idx, size_t(m.num_triangles) * 3 * sizeof(uint32_t));
         if (!e) s.mesh_buffers.push_back(idx);
         if (!e) e = hipMemcpy(pos, m.positions, size_t(m.num_vertices) * 3 * sizeof(float), hipMemcpyHostToDevice);
         if (!e) e = hipMemcpy(idx, m.indices, size_t(m.num_triangles) * 3 * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -3221,9 +3222,9 @@ int32_t create_scene_instanced(mi_mesh const* meshes, uint32_t num_meshes,
     for (uint32_t k = 0; k < num_meshes; ++k) {
         s.mesh_vertices[k] = meshes[k].num_vertices;
     }
-    hipError_t e = hipMalloc(&s.mesh_geo, std::max<size_t>(1, num_meshes) * sizeof(Mesh_geometry));
-    if (!e) e = hipMalloc(&s.inst_o2w, o2w.size() * sizeof(float));
-    if (!e) e = hipMalloc(&s.inst_material, mats.size() * sizeof(uint32_t));
+    hipError_t e = device_malloc(&s.mesh_geo, std::max<size_t>(1, num_meshes) * sizeof(Mesh_geometry));
+    if (!e) e = device_malloc(&s.inst_o2w, o2w.size() * sizeof(float));
+    if (!e) e = device_malloc(&s.inst_material, mats.size() * sizeof(uint32_t));
     if (!e && num_meshes) e = hipMemcpy(s.mesh_geo, geo.data(), num_meshes * sizeof(Mesh_geometry), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(s.inst_o2w, o2w.data(), o2w.size() * sizeof(float), hipMemcpyHostToDevice);
     if (!e) e = hipMemcpy(s.inst_material, mats.data(), mats.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -3351,7 +3352,7 @@ int32_t RenderState::reserve(uint32_t n, uint32_t num_shadow) {
         hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
         if (!e) e = hipEventCreateWithFlags(&begin, hipEventDisableTiming);
         if (!e) e = hipEventCreateWithFlags(&end, hipEventDisableTiming);
-        if (!e) e = hipMalloc(&counters, Num_counters * sizeof(uint32_t));
+        if (!e) e = device_malloc(&counters, Num_counters * sizeof(uint32_t));
         if (e) {
             release();
             return fail(MI_ERR_HIP, "render state: %s", hipGetErrorString(e));
@@ -3370,10 +3371,10 @@ int32_t RenderState::reserve(uint32_t n, uint32_t num_shadow) {
         occluded        = nullptr;
         picks           = nullptr;
         shadow_capacity = 0;
-        hipError_t e    = hipMalloc(&shadow_rays, size_t(num_shadow) * sizeof(mi_ray));
-        if (!e) e = hipMalloc(&shadows, size_t(num_shadow) * sizeof(Shadow));
-        if (!e) e = hipMalloc(&occluded, size_t(num_shadow) * sizeof(uint32_t));
-        if (!e) e = hipMalloc(&picks, size_t(num_shadow) * sizeof(Pick_slot));
+        hipError_t e    = device_malloc(&shadow_rays, size_t(num_shadow) * sizeof(mi_ray));
+        if (!e) e = device_malloc(&shadows, size_t(num_shadow) * sizeof(Shadow));
+        if (!e) e = device_malloc(&occluded, size_t(num_shadow) * sizeof(uint32_t));
+        if (!e) e = device_malloc(&picks, size_t(num_shadow) * sizeof(Pick_slot));
         if (e) {
             return fail(MI_ERR_HIP, "shadow queue of %u rays: %s", num_shadow, hipGetErrorString(e));
         }
@@ -3393,19 +3394,19 @@ int32_t RenderState::reserve(uint32_t n, uint32_t num_shadow) {
     (void)hipFree(medium_p);
     (void)hipFree(nee);
     capacity     = 0;
-    hipError_t e = hipMalloc(&paths, size_t(n) * sizeof(Path));
+    hipError_t e = device_malloc(&paths, size_t(n) * sizeof(Path));
     for (int q = 0; q < 2 && !e; ++q) {
-        e = hipMalloc(&rays[q], size_t(n) * sizeof(mi_ray));
-        if (!e) e = hipMalloc(&ray_path[q], size_t(n) * sizeof(uint32_t));
+        e = device_malloc(&rays[q], size_t(n) * sizeof(mi_ray));
+        if (!e) e = device_malloc(&ray_path[q], size_t(n) * sizeof(uint32_t));
     }
     // room for the closest hits of either scene kind
     static_assert(sizeof(mi_instance_hit) >= sizeof(mi_hit));
-    if (!e) e = hipMalloc(&hits, size_t(n) * sizeof(mi_instance_hit));
+    if (!e) e = device_malloc(&hits, size_t(n) * sizeof(mi_instance_hit));
     inst_hits = reinterpret_cast<mi_instance_hit*>(hits);
-    if (!e) e = hipMalloc(&shadow_range, size_t(n) * sizeof(uint2));
-    if (!e) e = hipMalloc(&medium_event, size_t(n) * sizeof(uint32_t));
-    if (!e) e = hipMalloc(&medium_p, size_t(n) * 3 * sizeof(float));
-    if (!e) e = hipMalloc(&nee, size_t(n) * sizeof(Nee_vertex));
+    if (!e) e = device_malloc(&shadow_range, size_t(n) * sizeof(uint2));
+    if (!e) e = device_malloc(&medium_event, size_t(n) * sizeof(uint32_t));
+    if (!e) e = device_malloc(&medium_p, size_t(n) * 3 * sizeof(float));
+    if (!e) e = device_malloc(&nee, size_t(n) * sizeof(Nee_vertex));
     if (e) {
         release();
         return fail(MI_ERR_HIP, "render state of %u paths: %s", n, hipGetErrorString(e));
@@ -3476,8 +3477,8 @@ int32_t RenderState::reserve_spectral(uint32_t n, uint32_t num_shadow) {
         path_spec         = nullptr;
         nee_thr4          = nullptr;
         spectral_capacity = 0;
-        hipError_t e      = hipMalloc(&path_spec, size_t(n) * sizeof(float2));
-        if (!e) e = hipMalloc(&nee_thr4, size_t(n) * sizeof(float));
+        hipError_t e      = device_malloc(&path_spec, size_t(n) * sizeof(float2));
+        if (!e) e = device_malloc(&nee_thr4, size_t(n) * sizeof(float));
         if (e) {
             return fail(MI_ERR_HIP, "spectral state of %u paths: %s", n, hipGetErrorString(e));
         }
@@ -3487,7 +3488,7 @@ int32_t RenderState::reserve_spectral(uint32_t n, uint32_t num_shadow) {
         (void)hipFree(shadow_c4);
         shadow_c4                = nullptr;
         spectral_shadow_capacity = 0;
-        if (hipError_t const e = hipMalloc(&shadow_c4, size_t(num_shadow) * sizeof(float)); e) {
+        if (hipError_t const e = device_malloc(&shadow_c4, size_t(num_shadow) * sizeof(float)); e) {
             return fail(MI_ERR_HIP, "spectral shadow queue of %u rays: %s", num_shadow,
                         hipGetErrorString(e));
         }
@@ -3513,7 +3514,7 @@ int32_t RenderState::reserve_regeneration(uint64_t samples, uint32_t slots) {
         (void)hipFree(sample_rad);
         sample_rad      = nullptr;
         sample_capacity = 0;
-        if (hipError_t const e = hipMalloc(&sample_rad, samples * 3 * sizeof(float)); e) {
+        if (hipError_t const e = device_malloc(&sample_rad, samples * 3 * sizeof(float)); e) {
             return fail(MI_ERR_HIP, "sample buffer of %llu samples: %s", (unsigned long long)samples,
                         hipGetErrorString(e));
         }
@@ -3523,7 +3524,7 @@ int32_t RenderState::reserve_regeneration(uint64_t samples, uint32_t slots) {
         (void)hipFree(done);
         done          = nullptr;
         done_capacity = 0;
-        if (hipError_t const e = hipMalloc(&done, size_t(slots) * sizeof(uint32_t)); e) {
+        if (hipError_t const e = device_malloc(&done, size_t(slots) * sizeof(uint32_t)); e) {
             return fail(MI_ERR_HIP, "ended-path list of %u slots: %s", slots, hipGetErrorString(e));
         }
         done_capacity = slots;
@@ -3541,7 +3542,7 @@ int32_t RenderState::reserve_pixel_samples(uint64_t entries) {
     (void)hipFree(pixel_samples);
     pixel_samples         = nullptr;
     pixel_sample_capacity = 0;
-    if (hipError_t const e = hipMalloc(&pixel_samples, entries * sizeof(float2)); e) {
+    if (hipError_t const e = device_malloc(&pixel_samples, entries * sizeof(float2)); e) {
         return fail(MI_ERR_HIP, "pixel sample table (%llu): %s", (unsigned long long)entries,
                     hipGetErrorString(e));
     }
@@ -3559,9 +3560,9 @@ int32_t RenderState::reserve_guiding(uint32_t n, uint32_t records) {
         (void)hipFree(guide_mix);
         guide_x = guide_raw = guide_mix = nullptr;
         guide_capacity      = 0;
-        hipError_t e        = hipMalloc(&guide_x, size_t(n) * 9 * sizeof(float));
-        if (!e) e = hipMalloc(&guide_raw, size_t(n) * 32 * sizeof(float));
-        if (!e) e = hipMalloc(&guide_mix, size_t(n) * dev::Vmf_mixture::Stored * sizeof(float));
+        hipError_t e        = device_malloc(&guide_x, size_t(n) * 9 * sizeof(float));
+        if (!e) e = device_malloc(&guide_raw, size_t(n) * 32 * sizeof(float));
+        if (!e) e = device_malloc(&guide_mix, size_t(n) * dev::Vmf_mixture::Stored * sizeof(float));
         if (e) {
             return fail(MI_ERR_HIP, "guiding buffers of %u paths: %s", n, hipGetErrorString(e));
         }
@@ -3583,16 +3584,16 @@ int32_t RenderState::reserve_guiding(uint32_t n, uint32_t records) {
         rec_path        = nullptr;
         rec_block       = nullptr;
         record_capacity = 0;
-        hipError_t e    = hipMalloc(&train_x, size_t(records) * 9 * sizeof(float));
-        if (!e) e = hipMalloc(&shuf_x, size_t(records) * 9 * sizeof(float));
-        if (!e) e = hipMalloc(&shuf_dir, size_t(records) * 3 * sizeof(float));
-        if (!e) e = hipMalloc(&shuf_w, size_t(records) * sizeof(float));
-        if (!e) e = hipMalloc(&train_dir, size_t(records) * 3 * sizeof(float));
-        if (!e) e = hipMalloc(&train_w, size_t(records) * sizeof(float));
-        if (!e) e = hipMalloc(&rec_t, size_t(records) * 3 * sizeof(float));
-        if (!e) e = hipMalloc(&rec_r, size_t(records) * 3 * sizeof(float));
-        if (!e) e = hipMalloc(&rec_path, size_t(records) * sizeof(uint32_t));
-        if (!e) e = hipMalloc(&rec_block, size_t((records + 255) / 256) * sizeof(uint32_t));
+        hipError_t e    = device_malloc(&train_x, size_t(records) * 9 * sizeof(float));
+        if (!e) e = device_malloc(&shuf_x, size_t(records) * 9 * sizeof(float));
+        if (!e) e = device_malloc(&shuf_dir, size_t(records) * 3 * sizeof(float));
+        if (!e) e = device_malloc(&shuf_w, size_t(records) * sizeof(float));
+        if (!e) e = device_malloc(&train_dir, size_t(records) * 3 * sizeof(float));
+        if (!e) e = device_malloc(&train_w, size_t(records) * sizeof(float));
+        if (!e) e = device_malloc(&rec_t, size_t(records) * 3 * sizeof(float));
+        if (!e) e = device_malloc(&rec_r, size_t(records) * 3 * sizeof(float));
+        if (!e) e = device_malloc(&rec_path, size_t(records) * sizeof(uint32_t));
+        if (!e) e = device_malloc(&rec_block, size_t((records + 255) / 256) * sizeof(uint32_t));
         if (e) {
             return fail(MI_ERR_HIP, "training records (%u): %s", records, hipGetErrorString(e));
         }

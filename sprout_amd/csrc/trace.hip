@@ -34,6 +34,7 @@
 
 #include "common.hpp"
 #include "device_math.hpp"
+#include "device_memory.hpp"
 #include "claims.hpp"
 #include "trace.hpp"
 
@@ -973,8 +974,8 @@ int32_t ensure_quantized(DeviceBvh const& bvh, hipStream_t stream) {
     }
     uint4*     q    = nullptr;
     uint32_t*  flag = nullptr;
-    hipError_t e    = hipMalloc(&q, size_t(num_pairs) * 2 * sizeof(uint4));
-    if (!e) e = hipMalloc(&flag, sizeof(uint32_t));
+    hipError_t e    = device_malloc(&q, size_t(num_pairs) * 2 * sizeof(uint4));
+    if (!e) e = device_malloc(&flag, sizeof(uint32_t));
     uint32_t odd = 1;
     if (!e) e = hipMemcpyAsync(flag, &odd, sizeof(uint32_t), hipMemcpyHostToDevice, stream);
     if (e) {
@@ -1112,8 +1113,8 @@ int32_t launch(DeviceBvh const& bvh, TraceResources& res, mi_ray const* rays, ui
                 nullptr, bytes, static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr),
                 static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr), int(num_rays), 0,
                 30, stream);
-            if (!e) e = hipMalloc(&res.sort_keys, 4 * size_t(num_rays) * sizeof(uint32_t));
-            if (!e) e = hipMalloc(&res.sort_temp, std::max<size_t>(bytes, 1));
+            if (!e) e = device_malloc(&res.sort_keys, 4 * size_t(num_rays) * sizeof(uint32_t));
+            if (!e) e = device_malloc(&res.sort_temp, std::max<size_t>(bytes, 1));
             if (e) {
                 return fail(MI_ERR_HIP, "ray order of %u rays: %s", num_rays, hipGetErrorString(e));
             }
