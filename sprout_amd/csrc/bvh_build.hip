@@ -80,6 +80,7 @@ constexpr uint32_t Err_index        = 2;
 constexpr uint32_t Err_layout       = 8;
 constexpr uint32_t Not_finite       = 16;  // no error: an instance's box is not finite
 constexpr uint32_t Err_capacity     = 32;  // a list or buffer is full: the host starts over with more
+constexpr uint32_t Err_level        = 8;   // from this bit on: the level of an unsplittable node
 constexpr uint32_t Err_stop         = Err_unsplittable | Err_index | Err_capacity;
 
 // scene::bvh::Reference: {min.xyz, primitive}{max.xyz, pad}
@@ -470,7 +471,6 @@ struct Build {
 constexpr uint32_t Counter_nodes = Num_lc * Kind_words;  // word offsets
 constexpr uint32_t Counter_leafs = Counter_nodes + Line;
 constexpr uint32_t Counter_error = Counter_nodes + 2 * Line;
-constexpr uint32_t Counter_level = Counter_error + 1;  // of an unsplittable node
 constexpr uint32_t Build_words = Counter_nodes + 3 * Line;
 
 __device__ __forceinline__ uint32_t* counter(Build const& b, uint32_t level, uint32_t which) {
@@ -492,10 +492,9 @@ __device__ __forceinline__ bool stopped(Build const& b) {
     return 0 != (error & Err_stop);
 }
 
-// The levels after one with such a node are not built: one level writes here.
+// The levels after one with such a node are not built: the level is one.
 __device__ __forceinline__ void unsplittable(Build const& b, uint32_t level) {
-    *counter(b, Counter_level) = level;
-    atomicOr(counter(b, Counter_error), Err_unsplittable);
+    atomicOr(counter(b, Counter_error), Err_unsplittable | level << Err_level);
 }
 
 __device__ __forceinline__ uint32_t bin_words(Build const& b) {
@@ -1241,10 +1240,7 @@ wave_nodes(Build b, uint32_t level) {
                 decide(t, axis, x, spatial, p, mine.cost, d);
                 needs_of(b.s, t, d, need);
                 if (0 == lane) {
-                    decision_s[i] = d;
-                    if (Kind_error == d.kind) {
-                        unsplittable(b, level);
-                    }
+                    decision_s[i] = d;  // a leaf or a split: up to 255 references are never unsplittable
                 }
             }
             if (0 == lane) {
@@ -1273,9 +1269,6 @@ wave_nodes(Build b, uint32_t level) {
                 continue;
             }
             Decision const d = decision_s[i];
-            if (Kind_leaf != d.kind && Kind_split != d.kind) {
-                continue;
-            }
             Task const     t = b.wave_tasks[level & 1][base + i];
             uint32_t const n = t.count;
             uint32_t       at[Num_needs];
@@ -2001,7 +1994,7 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
             return fail(MI_ERR_UNSPLITTABLE,
                         "mi_bvh_build: a node of more than 255 references cannot be split "
                         "(level %u)",
-                        host[Counter_level]);
+                        err >> Err_level);
         }
         if (err & Err_capacity) {
             continue;
