@@ -11,10 +11,14 @@ Workload (the reference's BVH micro-benchmark configuration):
           in HBM before the timed region)
 
 Prints one JSON line.  Secondary figures (coherent closest-hit, incoherent
-any-hit, build time) go into the same line.  The roofline object uses the
-reference loop's algorithmic bytes per ray (32 B per node fetched + 64 B per
-triangle test, counted on the GPU by the reference-order kernel on the same
-tree and rays) over the average kernel time measured with HIP events.
+any-hit, build time) go into the same line.  The kernel is bound by VALU issue:
+the roofline object sets the wave instructions of one step (the counter profile
+of this workload in profiles/) over the average kernel time measured with HIP
+events against four cycles of a SIMD each.  Beside it: the HBM traffic of the
+same profile as a share of HBM's peak, and the reference loop's algorithmic
+bytes per ray (32 B per node fetched + 64 B per triangle test, counted on the
+GPU by the reference-order kernel on the same tree and rays), which the caches
+serve.
 
     python bench.py [--steps K] [--warmup W] [--gpus 1]
 """
@@ -34,7 +38,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "trace_closest_c1.md")
+VALU_PEAK_GIPS = 256 * 4 * 2.4 / 4  # wave instructions: 1024 SIMDs at 2.4 GHz, four cycles each
+PROFILE_COUNTERS = os.path.join(ROOT, "profiles", "trace_closest_c1.md")
 
 
 def log(msg: str) -> None:
@@ -827,15 +832,22 @@ def main() -> int:
     torch.cuda.synchronize()
     cnt = cnt.cpu().numpy().astype(np.int64)
     alg_bytes = int(32 * cnt[:, 0].sum() + 64 * cnt[:, 1].sum())
-    achieved = alg_bytes / (ms_incoh * 1e-3) / 1e9
 
-    traffic = None
-    if os.path.exists(PROFILE_TRAFFIC):
+    traffic = instructions = lanes = None
+    if os.path.exists(PROFILE_COUNTERS):
         from sprout_amd.rocprof_summary import read_figures
 
-        prof = read_figures(PROFILE_TRAFFIC)
+        prof = read_figures(PROFILE_COUNTERS)
         if prof.get("num_rays") == n and prof.get("num_nodes") == info.num_nodes:
             traffic = prof.get("hbm_bytes_per_launch")
+            instructions = prof.get("SQ_INSTS_VALU")
+            lanes = prof.get("valu_lanes")
+
+    def per_second(count):
+        return None if count is None else count / (ms_incoh * 1e-3) / 1e9
+
+    achieved = per_second(instructions)
+    hbm = per_second(traffic)
 
     cpu = None
     if not args.no_cpu_baseline:
@@ -867,13 +879,16 @@ def main() -> int:
             "launch_shape": shape,
         },
         "roofline": {
-            "bound": "hbm",
-            "achieved": round(achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "bound": "valu_issue",
+            "achieved": achieved and round(achieved, 1),
+            "peak": VALU_PEAK_GIPS,
+            "unit": "G wave instructions/s",
+            "frac": achieved and round(achieved / VALU_PEAK_GIPS, 4),
+            "active_lanes_of_64": lanes,
             "traffic": traffic,
+            "hbm_frac": hbm and round(hbm / HBM_PEAK_GBS, 4),
             "algorithmic_bytes_per_ray": round(alg_bytes / n, 1),
+            "algorithmic_gbs": round(per_second(alg_bytes), 1),
             "kernel_ms": round(ms_incoh, 4),
         },
         "cpu_baseline": cpu,

@@ -15,10 +15,16 @@ are the 2nd .. (1 + W + S)th closest-hit dispatches (the 1st traces the
 camera rays).
 
     python -m sprout_amd.rocprof_summary <kt> <fetch> <write> <l2> --steps S --warmup W \
-        --rays N --nodes M --out profiles/trace_closest_c1.md --command "<the rocprofv3 lines>"
+        [--pmc <dir>...] --rays N --nodes M --out profiles/trace_closest_c1.md \
+        --command "<the rocprofv3 lines>"
+
+--pmc: further counter runs; the mean of each counter over the timed launches,
+and from SQ_INSTS_VALU, SQ_ACTIVE_INST_VALU, SQ_THREAD_CYCLES_VALU and
+GRBM_GUI_ACTIVE the share of the VALU issue cycles taken (a wave instruction
+takes a SIMD four cycles) and the lanes at work in one.
 
 The summary ends with "key: value" figures that bench.py reads for the
-roofline's `traffic` (only when its workload matches rays and nodes).
+roofline (only when its workload matches rays and nodes).
 """
 
 from __future__ import annotations
@@ -99,6 +105,27 @@ def summarize(kt, fetch, write, l2, steps, warmup, kernel=KERNEL):
         "l2_hit_rate": sum(hit) / (sum(hit) + sum(miss)),
     }
     return stats
+
+
+SIMDS = 1024
+XCCS = 8  # GRBM_GUI_ACTIVE reads the sum over them
+
+
+def timed_counters(dirs, kernel, steps, warmup):
+    """Mean per timed launch of every counter of the runs, and what follows."""
+    out = {}
+    for d in dirs:
+        rows = _rows(d, "counter_collection.csv")
+        for c in sorted({r["Counter_Name"] for r in rows}):
+            values = [v for _, v in _counter(rows, kernel, c)][slice(1, 1 + warmup + steps)]
+            if values:
+                out[c] = statistics.mean(values)
+    cycles = out.get("GRBM_GUI_ACTIVE", 0.0) / XCCS
+    if cycles and "SQ_ACTIVE_INST_VALU" in out:
+        out["valu_busy"] = 4 * out["SQ_ACTIVE_INST_VALU"] / (cycles * SIMDS)
+    if out.get("SQ_ACTIVE_INST_VALU") and "SQ_THREAD_CYCLES_VALU" in out:
+        out["valu_lanes"] = out["SQ_THREAD_CYCLES_VALU"] / out["SQ_ACTIVE_INST_VALU"]
+    return out
 
 
 def kernel_table(kt, top=12):
@@ -270,8 +297,10 @@ def main():
     ap.add_argument("--command", default="")
     ap.add_argument("--title", default="closest-hit traversal, BVH micro-benchmark")
     ap.add_argument("--kernel", default=KERNEL)
+    ap.add_argument("--pmc", nargs="*", default=[])
     args = ap.parse_args()
     s = summarize(args.kt, args.fetch, args.write, args.l2, args.steps, args.warmup, args.kernel)
+    s.update(timed_counters(args.pmc, args.kernel, args.steps, args.warmup))
     s["num_rays"] = args.rays
     s["num_nodes"] = args.nodes
     figures = "\n".join(f"{k}: {v:.6g}" if isinstance(v, float) else f"{k}: {v}"
