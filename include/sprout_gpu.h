@@ -100,7 +100,9 @@ char const* mi_last_error(void);
  * (>= 3), indices = num_triangles x 3 uint32.  The tree is the one
  * scene::shape::triangle::bvh::Builder_SAH::build produces
  * (triangle_bvh_builder_sah.cpp:21-67, scene_bvh_builder_base.cpp:26-290):
- * same nodes, same depth-first layout, same leaf order.  Synchronous.
+ * same nodes, same depth-first layout, same leaf order.  A triangle with a
+ * vertex that is not finite, which no ray hits, is in the tree with the box of
+ * its finite coordinates.  Synchronous.
  */
 int32_t mi_bvh_build(float const* positions, uint32_t num_vertices, uint32_t position_stride,
                      uint32_t const* indices, uint32_t num_triangles,

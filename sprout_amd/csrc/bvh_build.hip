@@ -1937,7 +1937,7 @@ int32_t build_bvh(float const* positions, uint32_t num_vertices, uint32_t positi
 
         size_t const bins_lds  = size_t(words) * sizeof(uint32_t);
         size_t const block_lds = Chunk * sizeof(Ref) + bins_lds;
-        // sets of bins of a workgroup within 48 KB: sixteen with 16 slices
+        // sets of bins of a workgroup within 48 KB: fifteen with 16 slices
         uint32_t const copies  = uint32_t(std::clamp<size_t>(48 * 1024 / bins_lds, 1, 16));
 
         // The host reads the lists' lengths once every few levels; until then

@@ -743,10 +743,9 @@ __device__ __forceinline__ dev::Channel_cc<4> wavelength_channels(dev::Medium_vi
 // later ones.
 // A frame of a 256^3 cloud, 512x512x4 paths: 3.81 ms with nested loops, 3.14
 // ms with the steps, 2.93 ms with each cell's leaf fetched a step ahead
-// (dev::Walk::next).  Workgroups a CU and rays a claim, before the last: 8 and
-// 64 took 3.32 ms a frame, 4 and 64
-// 3.20 ms, 4 and 16 3.12 ms, 2 and 16 3.41 ms; 8 to 48 service lanes are
-// within 1 %.
+// (dev::Walk::next).  Before that fetch a frame took, by workgroups a CU and
+// items a claim, 3.32 ms with 8 and 64, 3.20 ms with 4 and 64, 3.12 ms with 4
+// and 16, and 3.41 ms with 2 and 16; 8 to 48 service lanes are within 1 %.
 constexpr uint32_t Service_lanes = 16;
 constexpr uint32_t Walk_blocks   = 4;   // workgroups a CU
 constexpr uint32_t Walk_batch    = 16;  // items a claim

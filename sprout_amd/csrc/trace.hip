@@ -690,14 +690,16 @@ __device__ __forceinline__ bool inner_step_q(Launch const& p, Stack2& stack, Ray
 // ray's sign decide it), and the triangles are tested in the same relative
 // order.
 //
-// Incoherent rays are bound by VALU issue at few active lanes (4.2 M bounce
-// rays over 1.41 M triangles: 1.28e9 wave instructions in 2.40 ms at 21.7 of
-// 64 lanes, when every lane was taken down to a leaf before any leaf was
-// tested).  So a turn of the loop is one step of one kind, the kind that most
+// Incoherent rays are bound by VALU issue at few active lanes: 4.2 M bounce
+// rays over 1.41 M triangles took 1.28e9 wave instructions at 21.7 of 64 lanes
+// and 2.40 ms when every lane was taken down to a leaf before any leaf was
+// tested.  So a turn of the loop is one step of one kind, the kind that most
 // of the wave's lanes wait for: a sibling pair for the lanes at inner nodes,
-// or one triangle for the lanes at leaves (1.84 ms; thresholds of 8 to 32
-// lanes before a change of kind: 2.06 to 1.92).  Pops of both kinds share one
-// loop, and the children's boxes go through slab_lean.
+// or one triangle for the lanes at leaves.  Pops of both kinds share one loop,
+// and the children's boxes go through slab_lean: 8.1e8 instructions at 27.7
+// lanes in 1.55 to 1.72 ms, 86 % of the SIMDs' issue cycles.  Waiting for 8 to
+// 32 lanes of the other kind before a change, instead of for the majority,
+// took 4 to 12 % longer.
 template <bool Any, bool Quant>
 __global__ void trace_refill_packed(Launch p) {
     extern __shared__ uint32_t lds_stack[];

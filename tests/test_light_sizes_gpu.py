@@ -1,9 +1,10 @@
 """The device light-tree builder at the sizes where its kernels change path,
-against the host builder byte for byte: roots one thread folds and roots a
-workgroup folds (64, 65 lights), sweeps of more candidates than a workgroup
-has threads (85 and 86 lights: 255 and 258), sweep and grid (127, 128), LDS
-tiles of 256 lights, lights in one plane (infinite costs), duplicated lights
-(equal costs) and a tree deep enough that its levels' bounds start over."""
+against the host builder byte for byte: a wave folds 64 lights at a time (63
+to 65, and last chunks whose powers end inside a group of eight), the split's
+workgroup takes 256 candidates (85 and 86 lights: 255 and 258) and 256 lights
+(255 to 257, 513) a pass, sweep and grid (127, 128), lights in one plane
+(infinite costs), duplicated lights (equal costs), lights without power, and
+a tree deep enough that its levels' bounds start over (64)."""
 
 import numpy as np
 import pytest
