@@ -3952,8 +3952,9 @@ int32_t render(RenderScene const& scene, TraceResources& trace, float const* e_t
 
     // what the kernels of a bounce hold when they are captured
     auto bounce_key = [&]() -> Launch_key {
-        Launch_key key(sizeof(Wave));
-        std::memcpy(key.data(), &w, sizeof(Wave));
+        Launch_key key;
+        key.reserve(sizeof(Wave) + 512);  // one allocation
+        put_key(key, w);
         put_key(key, grid_path, num_shadow);
         put_trace_key(key, scene.bvh, trace);
         put_instances_key(key, scene.tlas);
